@@ -166,17 +166,17 @@ int sunhip_q_coefficients(sunhip_grid *g);
  * (0: last block finishes the dot products, 1: a finisher kernel), "tiles"
  * (tiles of 64 columns per block of the iteration's operator kernel: 4, 8,
  * 16), "ntstore" (1: its results stored with the non-temporal hint), "rzid"
- * (1: the preconditioned residual dot r.M^-1 r taken as sum d'^2/b' from
+ * (1: the preconditioned residual dot r.M^-1 r taken as sum d^2/b from
  * the forward Thomas sweep, so the backward sweep does not re-read r;
  * M^-1 r itself is unchanged), "minwaves" (register budget of the
  * operator kernel: 3 or 4 waves per SIMD; 0 the compiler's choice),
  * "blocklds" (1: the operator's neighbour values staged in LDS per block of
  * four tiles walking the levels together), "band" (levels per workgroup of
  * the operator kernel, 8 or more; 0 whole columns), "prec_head" (top levels
- * of each column whose Thomas pivots and forward values the preconditioner
- * keeps in registers between its sweeps: 0, 8, 16, 24, 32; -1, the
- * default: 24 from 1024 tiles of 64 columns up in FP64, 16 from 2048 tiles
- * up in FP32, else 0), "zreg" (1, the default: the
+ * of each column whose rows the preconditioner keeps in registers between
+ * its sweeps: 0, 8, 16, 24, 32; -1, the default: 40 in FP64 and 48 in FP32
+ * with the next 16 in LDS, from 1024 tiles of 64 columns up in FP64 and 2048
+ * in FP32, else 0), "zreg" (1, the default: the
  * z-level windows of sunhip_set_dz; 0 off), "order" (1, the default: blocks
  * of four tiles dispatched deepest first within each XCD's run; 0 in tile
  * order), "xchg" (the iteration's operator kernel exchanges neighbour values

@@ -130,18 +130,16 @@ __global__ __launch_bounds__(256) void kb_qprec(const BQMember<T, T> *__restrict
                                                 int nwork, double *__restrict__ part) {
   const int l = threadIdx.x & 63, stride = gridDim.x * BW;
   // each lane's rows of the LDS stage (its own words only)
-  constexpr int KL = 12;
-  __shared__ T lrows[3 * KL * 256];
+  constexpr int KL = QHead<T>::lds;
+  __shared__ T lrows[2 * KL * 256];
   for (int w = first_item(); w < nwork; w += stride) {
     const int2 it = W[w];
     const int m = __builtin_amdgcn_readfirstlane(it.x), t = __builtin_amdgcn_readfirstlane(it.y);
     const BQMember<T, T> &B = M[m];
     if (B.sc->done) continue;
     double rz = 0, rr = 0;
-    // the top 24 (FP64) or 16 (FP32) levels of each column stay in registers
-    // between the Thomas sweeps and the next 12 in LDS, as in the
-    // single-grid kernel
-    qprec_tile<true, U, T, true, sizeof(T) == 8 ? 24 : 16, false, KL>(B.G, B.coef, B.z, B.r, B.rtmp, B.bq,
+    // the register head and LDS stage of the single-grid kernel
+    qprec_tile<true, U, T, true, QHead<T>::regs, false, KL>(B.G, B.coef, B.z, B.r, B.rtmp, B.bq,
                                                                       (T)B.sc->nu, t, l, rz, rr, nullptr,
                                                                       lrows + threadIdx.x);
     rz = wave_sum(rz);

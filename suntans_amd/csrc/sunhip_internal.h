@@ -132,7 +132,7 @@ struct sunhip_grid {
   int *d_b4perm = nullptr;          // depth-first dispatch order of 4-tile blocks (Geo)
   int tune_order = 1;               // 1: use it
   int tune_tvdgrp = 2;              // levels per load group of the scalar column update (1, 2, 4)
-  int tune_plds = 12;               // levels below the preconditioner's register head kept in LDS (0, 12)
+  int tune_plds = 12;               // levels below a register head of 16 or 24 kept in LDS (0, 12)
   int tune_tvdhead = 8;             // rows of the scalar column update kept in registers (0, 8, 16)
   int tune_hblk = 1024;             // most blocks of the free-surface iteration kernels
   int tune_sumsgrp = 4;             // levels per load group of the TVD inflow sums (1, 2, 4)
@@ -217,9 +217,8 @@ struct sunhip_grid {
   int tune_xchg = -1;    // operator kernel with the neighbour exchange inside each wave: 0 off, 1 on,
                          // 2 on with a 4-waves-per-SIMD register budget, 3 on with 2 levels per group,
                          // -1 (default) 2 from 4096 tiles up, off below (short walks favour the plain kernel)
-  int tune_phead = -1;   // top levels per column the preconditioner keeps in registers (0, 8, 16, 24, 32;
-                         // FP32 solves use at most 16); -1 (default) 24 from 1024 tiles up in FP64, 16
-                         // from 2048 tiles up in FP32, 0 below
+  int tune_phead = -1;   // top levels per column the preconditioner keeps in registers (0, 8, 16, 24, 32);
+                         // -1 (default) QHead's from 1024 tiles up in FP64, 2048 in FP32, 0 below
   int tune_band = 0;     // operator kernel over level bands of this many levels (0: whole columns)
 
   // per-kernel timing (sunhip_profile): an event pair around every launch of

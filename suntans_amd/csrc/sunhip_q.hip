@@ -198,8 +198,8 @@ __global__ __launch_bounds__(256) void k_qprec(Geo G, const T *__restrict__ coef
                                                T *__restrict__ r, T *__restrict__ out, const T *__restrict__ bq,
                                                CGScal *sc, Red R, ZReg Z) {
   if (UPDATE && sc->done) return;
-  // rows of the LDS stage: [level][b', c, d'][lane of the block]
-  __shared__ T lrows[KL > 0 ? 3 * KL * 256 : 1];
+  // rows of the LDS stage: [level][e, l][lane of the block]
+  __shared__ T lrows[KL > 0 ? 2 * KL * 256 : 1];
   const int t = tile_group(G, blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6);
   double rz = 0, rr = 0;
   if (ZR && t < G.Nt && Z.tflag[t])
@@ -210,6 +210,12 @@ __global__ __launch_bounds__(256) void k_qprec(Geo G, const T *__restrict__ coef
                                                   threadIdx.x & 63, rz, rr, &Z, lrows + threadIdx.x);
   double v[2] = {rz, rr};
   reduce_out<2, 256>(v, R, sc);
+}
+
+__global__ __launch_bounds__(256) void k_qprec_ref(Geo G, const double *__restrict__ coef,
+                                                   const double *__restrict__ r, double *__restrict__ out,
+                                                   double *__restrict__ bq) {
+  qprec_ref_tile(G, coef, r, out, bq, blockIdx.x * 4 + (threadIdx.x >> 6), threadIdx.x & 63);
 }
 
 // qprecond=0: r -= nu*z, rtmp = r, alpha = eps = r.r (main/phys.c:2505-2519).
@@ -428,12 +434,18 @@ int launch_prec(sunhip_grid *g, CGScal *sc, const T *coef, const T *z, T *r, T *
     } \
   } while (0)
 #define PREC(U, KR) PREC3(U, KR, 0)
-  // FP32 columns keep 16 levels by default: 24 and 32 measured no faster on
-  // the 5e7-unknown solve (the register head costs occupancy)
+  // The default head and LDS stage (PREC3(4, 40, 16) / (4, 48, 16)): most
+  // columns of a 100-level grid then go through memory only once.  At 5e7
+  // unknowns heads of 24, 32, 40 and 48 levels with 16 in LDS take 460, 421,
+  // 390 and 467 us in FP64 (40: 2 waves per SIMD, 48 spills) and 231, 212,
+  // 219 and 207 us in FP32; without the LDS stage 32 levels take 485 and
+  // 248 us.  Few tiles (below 1024 in FP64, 2048 in FP32) take the plain
+  // sweep.
   const bool fp32 = std::is_same<T, float>::value;
-  int head = g->tune_phead;
-  if (head < 0) head = fp32 ? (g->Nt >= 2048 ? 16 : 0) : (g->Nt >= 1024 ? 24 : 0);
-  if (head == 0) {
+  const int head = g->tune_phead >= 0 ? g->tune_phead : (g->Nt >= (fp32 ? 2048 : 1024) ? 40 : 0);
+  if constexpr (!UPDATE) {
+    PREC(4, 0);  // once per solve; every variant gives the same bits
+  } else if (head == 0) {
     switch (g->tune_punroll) {
       case 1: PREC(1, 0); break;
       case 2: PREC(2, 0); break;
@@ -444,14 +456,15 @@ int launch_prec(sunhip_grid *g, CGScal *sc, const T *coef, const T *z, T *r, T *
     switch (head) {
       case 8: PREC(4, 8); break;
       case 16:
-        if (g->tune_plds == 12) PREC3(4, 16, 12);
+        if (g->tune_plds) PREC3(4, 16, 12);
         else PREC(4, 16);
         break;
       case 24:
-        if (g->tune_plds == 12) PREC3(4, 24, 12);
+        if (g->tune_plds) PREC3(4, 24, 12);
         else PREC(4, 24);
         break;
-      default: PREC(4, 32); break;
+      case 32: PREC(4, 32); break;
+      default: PREC3(4, QHead<T>::regs, QHead<T>::lds); break;
     }
   }
 #undef PREC
@@ -1089,9 +1102,8 @@ int sunhip_q_precondition(sunhip_grid *g, const char *x, const char *xc) {
   Field *fx, *fxc, *coef, *bq;
   int rc = field(g, x, &fx) | field(g, xc, &fxc) | field(g, "coef", &coef) | field(g, "qbp", &bq);
   if (rc) return rc;
-  if ((rc = launch_factor<double>(g, coef->d, bq->d))) return rc;
-  if ((rc = launch_prec<false, double>(g, g->d_qs, coef->d, nullptr, fx->d, fxc->d, bq->d, OP_NONE, nullptr)))
-    return rc;
+  k_qprec_ref<<<nb4(g), 256, 0, g->stream>>>(g->geo(), coef->d, fx->d, fxc->d, bq->d);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(g->stream));
   return 0;
 }

@@ -150,10 +150,24 @@ __device__ __forceinline__ void qcoef_tile(const Geo &G, const double *__restric
   }
 }
 
-// The modified diagonal b' of the Thomas elimination of every column
-// (main/util.c:193-196 applied to the tridiagonal of main/phys.c:3584-3601).
-// It depends only on coef, so it is built once per solve; the back
-// substitution of every application reads it.
+// One row of the vertical-line elimination of the solves.  The reference's
+// TriSolve (main/util.c:185-203) divides five times per level; here the
+// pivot is inverted once and the rest are products:
+//   b = diag - ck*l'       (ck = coef[k], l' = l of the row above)
+//   ib = 1/b ;  l = ck1*ib (ck1 = coef[k+1], 0 on the last level)
+//   d = r - l'*d' ;  e = d*ib ;  then upward u = e - l*u_below
+// The error has the bound of the reference's order (a few roundings per
+// level either way); OperatorQ's drop-in companion Preconditioner keeps the
+// reference's own order (qprec_ref_tile).
+template <typename T>
+__device__ __forceinline__ T q_pivot(int k, int kt, int n, T ck, T ck1, T lprev) {
+  T b = k == kt ? -2 * ck - ck1 : (k == n - 1 ? -ck : -ck - ck1);
+  if (k > kt) b = b - ck * lprev;
+  return T(1) / b;
+}
+
+// The inverse pivots ib of every column.  They depend only on coef, so they
+// are built once per solve.
 template <typename T>
 __device__ __forceinline__ void qfactor_tile(const Geo &G, const T *__restrict__ coef, T *__restrict__ bq, int t,
                                              int l) {
@@ -161,18 +175,15 @@ __device__ __forceinline__ void qfactor_tile(const Geo &G, const T *__restrict__
   const int s = t * 64 + l, n = G.nk[s], kt = G.ctop[s];
   if (n == 0 || G.comp[s] != 1 || kt >= n - 1) return;
   const int64_t base = G.toff[t] + l;
-  T cprev = 0, bprev = 1;
+  T lprev = 0;
   T ck = coef[base + (int64_t)kt * 64];
   for (int k = kt; k < n; k++) {
     const int64_t idx = base + (int64_t)k * 64;
     const T ck1 = k < n - 1 ? coef[idx + 64] : T(0);
-    T a = 0, b, c = 0;
-    if (k == kt) { b = -2 * ck - ck1; c = ck1; }
-    else if (k == n - 1) { a = ck; b = -ck; }
-    else { a = ck; b = -ck - ck1; c = ck1; }
-    if (k > kt) b -= a * cprev / bprev;
-    bq[idx] = b;
-    cprev = c; bprev = b; ck = ck1;
+    const T ib = q_pivot<T>(k, kt, n, ck, ck1, lprev);
+    bq[idx] = ib;
+    lprev = ck1 * ib;
+    ck = ck1;
   }
 }
 
@@ -195,6 +206,21 @@ __device__ __forceinline__ void st_stream(T *p, T v) {
   else *p = v;
 }
 
+// A column's share of a dot product, summed by segments of SUNHIP_SEG levels
+// (absolute level k / SUNHIP_SEG) and then over the segments from the top.
+// The kernels that walk a column with one lane and those that give each
+// segment a wave of its own (qapply_seg, qprec_seg) then add the same
+// values in the same order.
+#define SUNHIP_SEG 8
+struct SegSum {
+  double tot = 0, seg = 0;
+  __device__ __forceinline__ void add(int k, double v) {
+    if ((k & (SUNHIP_SEG - 1)) == 0) { tot += seg; seg = 0; }
+    seg += v;
+  }
+  __device__ __forceinline__ double sum() const { return tot + seg; }
+};
+
 // y = L v over the computational columns of tile t (main/phys.c:3486-3536),
 // in one of four modes:
 //   PLAIN     out = L vin
@@ -209,6 +235,7 @@ template <int MODE, int NF, int U, typename T, typename TO, bool NTS = false, bo
 __device__ __forceinline__ double qapply_tile(const Geo &G, const QVec<T, TO> &V, T mu, T nu, int t, int l,
                                               int k0 = 0, int k1 = 0x7fffffff) {
   double dot = 0;
+  SegSum ds;
   if (t >= G.Nt) return 0;
   const T *__restrict__ coef = V.coef;
   const T *__restrict__ dzf = V.dzf;
@@ -300,7 +327,7 @@ __device__ __forceinline__ double qapply_tile(const Geo &G, const QVec<T, TO> &V
         if (MODE == QM_FUSED) {
           st_stream<NTS>(&at32(V.pnew, idx), v0);
           st_stream<NTS>(&at32(V.x, idx), xv[j] + nu * pv[j]);
-          dot += (double)v0 * (double)y;
+          ds.add(k, (double)v0 * (double)y);
           st_stream<NTS, TO>(&at32(V.out, idx), (TO)y);
         } else if (MODE == QM_RESID) {
           at32(V.out, idx) = at32(V.src, idx) - y;
@@ -315,7 +342,7 @@ __device__ __forceinline__ double qapply_tile(const Geo &G, const QVec<T, TO> &V
     }
     vprev = v[U - 1];
   }
-  return dot;
+  return MODE == QM_FUSED ? ds.sum() : dot;
 }
 
 // ---- qprecond=1: the symmetrically scaled operator ------------------------
@@ -540,7 +567,7 @@ __device__ __forceinline__ double qapply_block(const Geo &G, const QVec<T, T> &V
     }
     lim[f] = kmx[f] > 0 ? kmx[f] - 1 : 0;
   }
-  double dot = 0;
+  SegSum ds;
   T vprev = 0;
   int buf = 0;
   for (int kb = kb0; kb < kb1; kb += U, buf ^= 1) {
@@ -603,14 +630,14 @@ __device__ __forceinline__ double qapply_block(const Geo &G, const QVec<T, T> &V
           const uint32_t idx = base + (uint32_t)k * 64u;
           st_stream<NTS>(&at32(V.pnew, idx), v0);
           st_stream<NTS>(&at32(V.x, idx), xv[j] + nu * pv[j]);
-          dot += (double)v0 * (double)y;
+          ds.add(k, (double)v0 * (double)y);
           st_stream<NTS>(&at32(V.out, idx), y);
         }
       }
     }
     vprev = v[U - 1];
   }
-  return dot;
+  return ds.sum();
 }
 
 // The FUSED mode of qapply_tile with the neighbour values exchanged inside
@@ -696,7 +723,7 @@ __device__ __forceinline__ double qapply_xchg(const Geo &G, const QVec<T, T> &V,
   }
   const bool two = np > 64;
   const int nn = n > 0 ? n : 0;
-  double dot = 0;
+  SegSum ds;
   T vprev = 0;
   for (int kb = kb0; kb < kb1; kb += U) {
     T v[U + 1], c[U + 1], pv[U + 1], xv[U], nv[U][NF], dz[U][NF], dzg[U];
@@ -768,14 +795,14 @@ __device__ __forceinline__ double qapply_xchg(const Geo &G, const QVec<T, T> &V,
           const uint32_t idx = base + (uint32_t)k * 64u;
           st_stream<NTS>(&at32(V.pnew, idx), v0);
           st_stream<NTS>(&at32(V.x, idx), xv[j] + nu * pv[j]);
-          dot += (double)v0 * (double)y;
+          ds.add(k, (double)v0 * (double)y);
           st_stream<NTS>(&at32(V.out, idx), y);
         }
       }
     }
     vprev = v[U - 1];
   }
-  return dot;
+  return ds.sum();
 }
 
 // qapply_xchg for a tile whose columns fit their z-level windows, software
@@ -833,7 +860,7 @@ __device__ __forceinline__ double qapply_xchg_pipe(const Geo &G, const QVec<T, T
     plim = mx > 0 ? mx - 1 : 0;
   }
   const int nn = n > 0 ? n : 0;
-  double dot = 0;
+  SegSum ds;
   T vprev = 0;
   // the loads of the group at kb (raw values; combined where used)
   auto load = [&](int kb, T (&pv)[U + 1], T (&v)[U + 1], T (&xv)[U], T (&r0)[U], T (&p0)[U], T (&dz)[U]) {
@@ -894,7 +921,7 @@ __device__ __forceinline__ double qapply_xchg_pipe(const Geo &G, const QVec<T, T
           const uint32_t idx = base + (uint32_t)k * 64u;
           st_stream<NTS>(&at32(V.pnew, idx), v0);
           st_stream<NTS>(&at32(V.x, idx), xv[j] + nu * pv[j]);
-          dot += (double)v0 * (double)y;
+          ds.add(k, (double)v0 * (double)y);
           st_stream<NTS>(&at32(V.out, idx), y);
         }
       }
@@ -911,25 +938,33 @@ __device__ __forceinline__ double qapply_xchg_pipe(const Geo &G, const QVec<T, T
     if (kb + 2 * U < kb1) load(kb + 2 * U, pvA, vA, xvA, r0A, p0A, dzA);
     process(kb + U, pvB, vB, xvB, r0B, p0B, dzB);
   }
-  return dot;
+  return ds.sum();
 }
 
 // Vertical-line preconditioner of tile t: (UPDATE) r -= nu*z, then
-// out = M^-1 r by Thomas down the column (b' recomputed, d' stored in out)
-// and back up it (b' from bq); rz and rr collect the lane's r.out and r.r.
-// RZID: rz from the forward sweep alone, r.M^-1 r = sum d'^2/b' (M = L D L^T
-// with D = diag(b') and d' = L^-1 r), so the backward sweep does not read r
+// out = M^-1 r down the column (e stored in out) and back up it; rz and rr
+// collect the lane's r.out and r.r.
+// RZID: rz from the forward sweep alone, r.M^-1 r = sum d*e (M = L D L^T with
+// D = diag(b), d = L^-1 r, e = d/b), so the backward sweep does not read r
 // again; out is unchanged, only the rounding of rz differs.
-// KR > 0: the top KR levels of the column keep b', d' and c in registers
-// between the sweeps (their backward step reads nothing and their d' never
-// goes to memory); the levels below go through out and bq as above.  The
+// KR > 0: the top KR levels of the column keep e and l in registers between
+// the sweeps (their backward step reads nothing and their e never goes to
+// memory); the levels below go through out and bq (the inverse pivots).  The
 // arithmetic and its order are the same for every KR.
 // ZR (a tile whose columns fit their z-level windows): coef formed from
 // the window and the exceptions (Z), as in qapply_tile.
-// KL > 0 (with KR > 0): the KL levels below the head keep b', c and d' in
-// LDS between the sweeps (lrow: this lane's first word, the block's lanes
-// interleaved, 3*KL words of stride 256), so they neither write d' to out
+// KL > 0 (with KR > 0): the KL levels below the head keep e and l in LDS
+// between the sweeps (lrow: this lane's first word, the block's lanes
+// interleaved, 2*KL words of stride 256), so they neither write e to out
 // nor read out, bq and coef back; the arithmetic is the same again.
+//
+// The head and LDS stage of the large solves: 4 registers (FP64) and two LDS
+// words per level, 256 VGPRs and 64 KB per block of four tiles, so two
+// blocks share a CU.
+template <typename T>
+struct QHead {
+  static constexpr int regs = sizeof(T) == 8 ? 40 : 48, lds = 16;
+};
 template <bool UPDATE, int U, typename T, bool RZID = false, int KR = 0, bool ZR = false, int KL = 0>
 __device__ __forceinline__ void qprec_tile(const Geo &G, const T *__restrict__ coef, const T *__restrict__ z,
                                            T *__restrict__ r, T *__restrict__ out, const T *__restrict__ bq, T nu,
@@ -943,6 +978,8 @@ __device__ __forceinline__ void qprec_tile(const Geo &G, const T *__restrict__ c
   const ZCol<T> zc = ZR ? zcol<T>(*Zp, G, s, kt, n) : ZCol<T>{};
   // coef at level k (k <= n; level n is never used but stays in the tile)
   auto C = [&](int k) -> T { return ZR ? zc.at(k) : at32(coef, base + (uint32_t)k * 64u); };
+  SegSum sz, sr;  // rz (RZID) and rr
+  double uz = 0;  // rz of the backward sweep
   if (kt == n - 1) {
     const uint32_t idx = base + (uint32_t)kt * 64u;
     T rk = at32(r, idx);
@@ -953,9 +990,24 @@ __device__ __forceinline__ void qprec_tile(const Geo &G, const T *__restrict__ c
     rr += (double)rk * (double)rk;
     return;
   }
+  T lprev = 0, dprev = 0;
+  // one level of the forward sweep: the loaded r, z and coef at k and k+1 in,
+  // e and l out
+  auto row = [&](int k, T rv, T zv, T ck, T cn, T &e, T &lk) -> T {
+    T rk = rv;
+    if (UPDATE) { rk = rk - nu * zv; st_stream<true>(&at32(r, base + (uint32_t)k * 64u), rk); }
+    sr.add(k, (double)rk * (double)rk);
+    const T ck1 = k == n - 1 ? T(0) : cn;
+    const T ib = q_pivot<T>(k, kt, n, ck, ck1, lprev);
+    const T d = rk - lprev * dprev;
+    e = d * ib;
+    lk = ck1 * ib;
+    if constexpr (RZID) sz.add(k, (double)d * (double)e);
+    lprev = lk; dprev = d;
+    return rk;
+  };
   constexpr int KH = KR > 0 ? KR : 1;
-  T hb[KH], hd[KH], hc[KH], hr[KH];
-  T cprev = 0, bprev = 1, dprev = 0;
+  T he[KH], hl[KH], hr[KH];
   if constexpr (KR > 0) {
     // the head in groups of HG levels: a group's loads (clamped into the
     // tile, which stores one level below its deepest column) are all issued
@@ -979,38 +1031,23 @@ __device__ __forceinline__ void qprec_tile(const Geo &G, const T *__restrict__ c
       for (int jj = 0; jj < HG; jj++) {
         const int j = g0 + jj, k = kt + j;
         if (k < n) {
-          const uint32_t idx = base + (uint32_t)k * 64u;
-          const T ck = cg[jj], ck1 = cg[jj + 1];
-          T rk = rg[jj];
-          if (UPDATE) { rk = rk - nu * zg[jj]; st_stream<true>(&at32(r, idx), rk); }
-          rr += (double)rk * (double)rk;
-          T a = 0, b, c = 0;
-          if (k == kt) { b = -2 * ck - ck1; c = ck1; }
-          else if (k == n - 1) { a = ck; b = -ck; }
-          else { a = ck; b = -ck - ck1; c = ck1; }
-          T d = rk;
-          if (k > kt) {
-            b -= a * cprev / bprev;
-            d -= a * dprev / bprev;
-          }
-          if constexpr (RZID) rz += (double)d * (double)d / (double)b;
-          hb[j] = b; hd[j] = d; hc[j] = c;
+          const T rk = row(k, rg[jj], zg[jj], cg[jj], cg[jj + 1], he[j], hl[j]);
           if constexpr (!RZID) hr[j] = rk;
-          cprev = c; bprev = b; dprev = d;
         }
       }
     }
   }
-  // the LDS stage: levels kt+KR .. kt+KR+KL-1, as the memory loop below but
-  // with the row kept in lrow
-  const int kls = kt + KR, kle = min(n, kt + KR + KL);
-  if constexpr (KL > 0) {
-    for (int kb = kls; kb < kle; kb += U) {
+  // the levels below the head, U at a time: first those of the LDS stage
+  // (kls .. kle-1), then those that go through memory (klo .. n-1)
+  const int kls = kt + KR, kle = min(n, kt + KR + KL), klo = kt + KR + KL;
+  auto sweep = [&](int k0, int k1, auto &&put) {
+    for (int kb = k0; kb < k1; kb += U) {
       T rv[U], zv[U], cv[U + 1];
 #pragma unroll
       for (int j = 0; j <= U; j++) {
-        const uint32_t idx = base + (uint32_t)min(kb + j, n) * 64u;
-        cv[j] = C(min(kb + j, n));
+        const int k = min(kb + j, n);
+        const uint32_t idx = base + (uint32_t)k * 64u;
+        cv[j] = C(k);
         if (j < U) {
           rv[j] = at32((const T *)r, idx);
           zv[j] = UPDATE ? at32(z, idx) : T(0);
@@ -1019,99 +1056,51 @@ __device__ __forceinline__ void qprec_tile(const Geo &G, const T *__restrict__ c
 #pragma unroll
       for (int j = 0; j < U; j++) {
         const int k = kb + j;
-        if (k < kle) {
-          const uint32_t idx = base + (uint32_t)k * 64u;
-          T rk = rv[j];
-          if (UPDATE) { rk = rk - nu * zv[j]; st_stream<true>(&at32(r, idx), rk); }
-          rr += (double)rk * (double)rk;
-          const T ck = cv[j], ck1 = cv[j + 1];
-          T a = 0, b, c = 0;
-          if (k == kt) { b = -2 * ck - ck1; c = ck1; }
-          else if (k == n - 1) { a = ck; b = -ck; }
-          else { a = ck; b = -ck - ck1; c = ck1; }
-          T d = rk;
-          if (k > kt) {
-            b -= a * cprev / bprev;
-            d -= a * dprev / bprev;
-          }
-          if constexpr (RZID) rz += (double)d * (double)d / (double)b;
-          T *w = lrow + (3 * (k - kls)) * 256;
-          w[0] = b;
-          w[256] = c;
-          w[512] = d;
-          cprev = c; bprev = b; dprev = d;
+        if (k < k1) {
+          T e, lk;
+          row(k, rv[j], zv[j], cv[j], cv[j + 1], e, lk);
+          put(k, e, lk);
         }
       }
     }
-  }
-  const int klo = kt + KR + KL;  // first level that goes through memory
-  for (int kb = klo; kb < n; kb += U) {
-    T rv[U], zv[U], cv[U + 1];
-#pragma unroll
-    for (int j = 0; j <= U; j++) {
-      const uint32_t idx = base + (uint32_t)min(kb + j, n) * 64u;
-      cv[j] = C(min(kb + j, n));
-      if (j < U) {
-        rv[j] = at32((const T *)r, idx);
-        zv[j] = UPDATE ? at32(z, idx) : T(0);
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < U; j++) {
-      const int k = kb + j;
-      if (k < n) {
-        const uint32_t idx = base + (uint32_t)k * 64u;
-        T rk = rv[j];
-        if (UPDATE) { rk = rk - nu * zv[j]; st_stream<true>(&at32(r, idx), rk); }
-        rr += (double)rk * (double)rk;
-        const T ck = cv[j], ck1 = cv[j + 1];
-        T a = 0, b, c = 0;
-        if (k == kt) { b = -2 * ck - ck1; c = ck1; }
-        else if (k == n - 1) { a = ck; b = -ck; }
-        else { a = ck; b = -ck - ck1; c = ck1; }
-        T d = rk;
-        if (k > kt) {
-          b -= a * cprev / bprev;
-          d -= a * dprev / bprev;
-        }
-        at32(out, idx) = d;
-        if constexpr (RZID) rz += (double)d * (double)d / (double)b;
-        cprev = c; bprev = b; dprev = d;
-      }
-    }
-  }
-  T unext = 0, cnext = 0;
+  };
+  if constexpr (KL > 0)
+    sweep(kls, kle, [&](int k, T e, T lk) {
+      T *w = lrow + (2 * (k - kls)) * 256;
+      w[0] = e;
+      w[256] = lk;
+    });
+  sweep(klo, n, [&](int k, T e, T) { at32(out, base + (uint32_t)k * 64u) = e; });
+  T unext = 0;
   for (int ke = n - 1; ke >= klo; ke -= U) {
-    T bv[U], dv[U], rv[U], cv[U];
+    T iv[U], ev[U], rv[U], cv[U];
 #pragma unroll
     for (int j = 0; j < U; j++) {
-      const uint32_t idx = base + (uint32_t)max(ke - j, klo) * 64u;
-      bv[j] = at32(bq, idx);
-      dv[j] = at32((const T *)out, idx);
+      const int k = max(ke - j, klo);
+      const uint32_t idx = base + (uint32_t)k * 64u;
+      iv[j] = at32(bq, idx);
+      ev[j] = at32((const T *)out, idx);
       rv[j] = RZID ? T(0) : at32((const T *)r, idx);
-      cv[j] = C(max(ke - j, klo));
+      cv[j] = k == n - 1 ? T(0) : C(k + 1);
     }
 #pragma unroll
     for (int j = 0; j < U; j++) {
       const int k = ke - j;
       if (k >= klo) {
-        const T b = bv[j], d = dv[j];
-        const T u = (k == n - 1) ? d / b : d / b - cnext * unext / b;
+        const T u = ev[j] - (cv[j] * iv[j]) * unext;
         st_stream<true>(&at32(out, base + (uint32_t)k * 64u), u);
-        if constexpr (!RZID) rz += (double)rv[j] * (double)u;
+        if constexpr (!RZID) uz += (double)rv[j] * (double)u;
         unext = u;
-        cnext = cv[j];  // c at level k-1 is coef[k]
       }
     }
   }
   if constexpr (KL > 0) {
     for (int k = kle - 1; k >= kls; k--) {
-      const T *w = lrow + (3 * (k - kls)) * 256;
-      const T b = w[0], c = w[256], d = w[512];
-      const T u = (k == n - 1) ? d / b : d / b - c * unext / b;
+      const T *w = lrow + (2 * (k - kls)) * 256;
+      const T u = w[0] - w[256] * unext;
       const uint32_t idx = base + (uint32_t)k * 64u;
       st_stream<true>(&at32(out, idx), u);
-      if constexpr (!RZID) rz += (double)at32((const T *)r, idx) * (double)u;
+      if constexpr (!RZID) uz += (double)at32((const T *)r, idx) * (double)u;
       unext = u;
     }
   }
@@ -1120,13 +1109,56 @@ __device__ __forceinline__ void qprec_tile(const Geo &G, const T *__restrict__ c
     for (int j = KR - 1; j >= 0; j--) {
       const int k = kt + j;
       if (k < n) {
-        const T b = hb[j], d = hd[j];
-        const T u = (k == n - 1) ? d / b : d / b - hc[j] * unext / b;
+        const T u = he[j] - hl[j] * unext;
         st_stream<true>(&at32(out, base + (uint32_t)k * 64u), u);
-        if constexpr (!RZID) rz += (double)hr[j] * (double)u;
+        if constexpr (!RZID) uz += (double)hr[j] * (double)u;
         unext = u;
       }
     }
+  }
+  rz += RZID ? sz.sum() : uz;
+  rr += sr.sum();
+}
+
+// Preconditioner as the reference orders it (main/phys.c:3577-3619 with
+// TriSolve): out = M^-1 r, bit for bit; the pivots b' go through bq.
+__device__ __forceinline__ void qprec_ref_tile(const Geo &G, const double *__restrict__ coef,
+                                               const double *__restrict__ r, double *__restrict__ out,
+                                               double *__restrict__ bq, int t, int l) {
+  if (t >= G.Nt) return;
+  const int s = t * 64 + l, n = G.nk[s], kt = G.ctop[s];
+  if (n == 0 || G.comp[s] != 1) return;
+  const uint32_t base = (uint32_t)(G.toff[t] + l);
+  if (kt == n - 1) {
+    const uint32_t idx = base + (uint32_t)kt * 64u;
+    at32(out, idx) = -0.5 * at32(r, idx) / at32(coef, idx);
+    return;
+  }
+  double cprev = 0, bprev = 1, dprev = 0;
+  double ck = at32(coef, base + (uint32_t)kt * 64u);
+  for (int k = kt; k < n; k++) {
+    const uint32_t idx = base + (uint32_t)k * 64u;
+    const double ck1 = k < n - 1 ? at32(coef, idx + 64u) : 0.0;
+    double a = 0, b, c = 0, d = at32(r, idx);
+    if (k == kt) { b = -2 * ck - ck1; c = ck1; }
+    else if (k == n - 1) { a = ck; b = -ck; }
+    else { a = ck; b = -ck - ck1; c = ck1; }
+    if (k > kt) {
+      b -= a * cprev / bprev;
+      d -= a * dprev / bprev;
+    }
+    at32(bq, idx) = b;
+    at32(out, idx) = d;
+    cprev = c; bprev = b; dprev = d; ck = ck1;
+  }
+  double un = dprev / bprev, cn = at32(coef, base + (uint32_t)(n - 1) * 64u);
+  at32(out, base + (uint32_t)(n - 1) * 64u) = un;
+  for (int k = n - 2; k >= kt; k--) {
+    const uint32_t idx = base + (uint32_t)k * 64u;
+    const double b = at32(bq, idx);
+    un = at32(out, idx) / b - cn * un / b;
+    at32(out, idx) = un;
+    cn = at32(coef, idx);  // c at level k-1 is coef[k]
   }
 }
 

@@ -1,0 +1,44 @@
+"""The preconditioner of the solves (inverse pivots, register head and LDS
+stage) at column depths around the ends of its stages: 40 + 16 levels in
+FP64, 48 + 16 in FP32.  The batched engine runs that head at every size; the
+single-grid solve with prec_head 0 runs the plain sweep.  Both form the same
+values, the engine summing its dot products per tile, so that q moves by
+roundings of the dots only: 1e-12."""
+import numpy as np
+import pytest
+
+from suntans_amd import cases, device
+
+pytestmark = pytest.mark.gpu
+
+
+def build(levels):
+    st = cases.tiny(levels, nx=11, ny=9, Nkmax=levels, min_layers=1)
+    dg = device.DeviceGrid(st)
+    device.member_upload(dg, st)
+    return st, dg
+
+
+@pytest.mark.parametrize("levels", [3, 39, 40, 41, 55, 56, 57, 63, 64, 65, 72])
+def test_head_against_plain_sweep(gpu_available, levels):
+    st, dg = build(levels)
+    n = dg.sizes()["Nflat"]
+    dg.tune("prec_head", 0)
+    s0 = dg.q_solve(epsilon=1e-10)
+    q0 = dg.download("q", n)
+    dg.upload("q", st.get("qc"))
+    b = device.Batch()
+    s1 = b.q_solve([dg], epsilon=1e-10)[0]
+    q1 = dg.download("q", n)
+    assert s0["converged"] and s1["converged"] and abs(s0["niters"] - s1["niters"]) <= 1
+    # one iteration more or less moves q by its residual; equal counts by roundings
+    tol = 1e-12 if s0["niters"] == s1["niters"] else 1e-8
+    assert np.linalg.norm(q1 - q0) <= tol * np.linalg.norm(q0)
+    dg.upload("q", st.get("qc"))
+    s2 = b.q_solve_mixed([dg], epsilon=1e-10, inner_tol=1e-4)[0]
+    q2 = dg.download("q", n)
+    b.close()
+    dg.close()
+    # both stop at a true residual of 1e-10
+    assert s2["converged"]
+    assert np.linalg.norm(q2 - q0) <= 1e-8 * np.linalg.norm(q0)
