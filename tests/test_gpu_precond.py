@@ -19,7 +19,7 @@ def build(levels):
     return st, dg
 
 
-@pytest.mark.parametrize("levels", [3, 39, 40, 41, 55, 56, 57, 63, 64, 65, 72])
+@pytest.mark.parametrize("levels", [5, 39, 40, 41, 55, 56, 57, 63, 64, 65, 72])
 def test_head_against_plain_sweep(gpu_available, levels):
     st, dg = build(levels)
     n = dg.sizes()["Nflat"]
