@@ -30,7 +30,7 @@ LIB = os.path.join(HERE, "lib")
 INC = os.path.join(ROOT, "include")
 OBJ = os.path.join(ROOT, "_build", "obj")
 
-HIP_SOURCES = ["sunhip_grid.hip", "sunhip_q.hip", "sunhip_h.hip", "sunhip_tvd.hip", "sunhip_batch.hip",
+HIP_SOURCES = ["sunhip_grid.hip", "sunhip_q.hip", "sunhip_qseg.hip", "sunhip_h.hip", "sunhip_tvd.hip", "sunhip_batch.hip",
                "sunhip_step.hip", "sunhip_upred.hip", "sunhip_vgrid.hip", "sunhip_wpred.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 HIPFLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",

@@ -85,6 +85,7 @@ sunhip::Geo sunhip_grid::geo() const {
   G.df = d_df; G.dg = d_dg;
   G.xcode = d_xcode; G.pair = d_pair; G.npair = d_npair;
   G.b4perm = tune_order ? d_b4perm : nullptr;
+  G.b4inv = d_b4inv;
   return G;
 }
 
@@ -416,6 +417,7 @@ int sunhip_grid_create(sunhip_grid **out, const sunhip_topology *T, int device) 
   }
   for (int ip = T->celldist[0]; ip < T->celldist[1]; ip++) comp[g->slot_of_cell[T->cellp[ip]]] = 1;
   for (int ip = T->celldist[1]; ip < T->celldist[2]; ip++) comp[g->slot_of_cell[T->cellp[ip]]] = 2;
+  g->has_bnd = T->celldist[1] - T->celldist[0] < g->Nc;
   std::vector<int> ec1(NES, -1), ec2(NES, -1), es1(NES, -1), es2(NES, -1), enkc(NES, 0), emark(NES, 0),
       ecomp(NES, 0);
   std::vector<double> df(NES, 0.0), dg(NES, 0.0);
@@ -536,16 +538,23 @@ int sunhip_grid_create(sunhip_grid **out, const sunhip_topology *T, int device) 
       start += len;
     }
     rc |= upload_vec(g, &g->d_b4perm, perm);
+    // block v works on group perm[u], u the v-th block's place in its XCD's run
+    std::vector<int> inv(nb4);
+    for (int v = 0; v < nb4; v++) {
+      const int x = v & 7, u = x * q + std::min(x, r8) + (v >> 3);
+      inv[perm[u]] = v;
+    }
+    rc |= upload_vec(g, &g->d_b4inv, inv);
   }
   rc |= upload_vec(g, &g->d_e_nke, ezeros);
   rc |= upload_vec(g, &g->d_e_etop, ezeros);
   rc |= upload_vec(g, &g->d_e_etopold, ezeros);
   // reductions: one partial pair per block of the widest launch
   const int nblk = std::max(g->Nt, g->Net) + 64;
-  g->part_n = 4 * (int64_t)nblk;
+  g->part_n = std::max<int64_t>(4 * (int64_t)nblk, 16 * (int64_t)((g->Nt + 3) / 4));
   rc |= dev_alloc(g, (void **)&g->d_part, sizeof(double) * (size_t)g->part_n);
   rc |= dev_alloc(g, (void **)&g->d_count, sizeof(unsigned) * 64);
-  rc |= dev_alloc(g, (void **)&g->d_qs, sizeof(CGScal));
+  rc |= dev_alloc(g, (void **)&g->d_qs, 2 * sizeof(CGScal));
   rc |= dev_alloc(g, (void **)&g->d_hs, 2 * sizeof(CGScal));  // two: the free-surface iteration alternates them
   rc |= dev_alloc(g, (void **)&g->d_ms, 2 * sizeof(CGScal));
   rc |= dev_alloc(g, (void **)&g->d_mo, sizeof(CGScal));
@@ -553,6 +562,8 @@ int sunhip_grid_create(sunhip_grid **out, const sunhip_topology *T, int device) 
   HIPCHK(hipMemset(g->d_count, 0, sizeof(unsigned) * 64));
   HIPCHK(hipHostMalloc((void **)&g->h_sc, sizeof(CGScal), hipHostMallocDefault));
   HIPCHK(hipHostMalloc((void **)&g->h_poll, 2 * sizeof(CGScal), hipHostMallocDefault));
+  HIPCHK(hipHostMalloc((void **)&g->h_prog, sizeof(unsigned long long), hipHostMallocDefault));
+  *g->h_prog = 0;
   HIPCHK(hipEventCreateWithFlags(&g->evp[0], hipEventDisableTiming));
   HIPCHK(hipEventCreateWithFlags(&g->evp[1], hipEventDisableTiming));
   HIPCHK(hipEventCreate(&g->ev0));
@@ -578,7 +589,7 @@ int sunhip_grid_destroy(sunhip_grid *g) {
                   g->d_e_etop, g->d_e_mark, g->d_e_comp, g->d_cstart, g->d_cstartw, g->d_estart,
                   g->d_cellslot, g->d_edgeslot, g->d_stage[0], g->d_stage[1], g->d_stage[2], g->d_stage[3], g->d_part, g->d_count, g->d_qs, g->d_hs,
                   g->d_class_tiles, g->d_ms, g->d_mo, g->d_D32, g->d_h32, g->d_uerr, g->d_dz, g->d_e_etopold,
-                  g->d_ford, g->d_zdzt, g->d_cwin, g->d_fwin, g->d_cex, g->d_fex, g->d_tflag, g->d_b4perm};
+                  g->d_ford, g->d_zdzt, g->d_cwin, g->d_fwin, g->d_cex, g->d_fex, g->d_tflag, g->d_b4perm, g->d_b4inv};
   for (void *p : ptrs) if (p) hipFree(p);
   for (int i = 0; i < SUNHIP_PIN_SLOTS; i++) {
     if (g->h_pin[i]) hipHostFree(g->h_pin[i]);
@@ -594,6 +605,7 @@ int sunhip_grid_destroy(sunhip_grid *g) {
   if (g->xdown) hipStreamDestroy(g->xdown);
   if (g->h_sc) hipHostFree(g->h_sc);
   if (g->h_poll) hipHostFree(g->h_poll);
+  if (g->h_prog) hipHostFree(g->h_prog);
   for (hipEvent_t e : g->evp) if (e) hipEventDestroy(e);
   if (g->ev0) hipEventDestroy(g->ev0);
   if (g->ev1) hipEventDestroy(g->ev1);

@@ -103,6 +103,8 @@ struct Geo {
   // deepest go first, so the launch does not end on a few deep columns;
   // null: identity
   const int *b4perm;
+  // the inverse: b4inv[g] = the block whose group tile_group gives as g
+  const int *b4inv;
 };
 
 }  // namespace sunhip
@@ -130,6 +132,7 @@ struct sunhip_grid {
   int *d_nbb = nullptr, *d_nbs = nullptr, *d_eb = nullptr, *d_es = nullptr, *d_nrm = nullptr, *d_kr = nullptr;
   int *d_xcode = nullptr, *d_pair = nullptr, *d_npair = nullptr;  // neighbour exchange (Geo)
   int *d_b4perm = nullptr;          // depth-first dispatch order of 4-tile blocks (Geo)
+  int *d_b4inv = nullptr;           // its inverse (Geo)
   int tune_order = 1;               // 1: use it
   int tune_tvdgrp = 2;              // levels per load group of the scalar column update (1, 2, 4)
   int tune_plds = 12;               // levels below a register head of 16 or 24 kept in LDS (0, 12)
@@ -152,6 +155,7 @@ struct sunhip_grid {
   int n_type4 = 0;                   // no-slip (type-4) edges
   int type2_ok = 1;                  // every type-2 edge has its cell on the grad[2j] side
   bool have_def1 = false;            // "def1" holds the face distances (sunhip_set_face_distances)
+  bool has_bnd = false;              // columns that are not computational
   int max_pairs = 0;                 // most cross-tile faces of any tile
   double *d_Ac = nullptr, *d_df = nullptr, *d_dg = nullptr;
   int *d_e_c1 = nullptr, *d_e_c2 = nullptr, *d_e_s1 = nullptr, *d_e_s2 = nullptr;
@@ -196,6 +200,8 @@ struct sunhip_grid {
   sunhip::CGScal *d_ms = nullptr, *d_mo = nullptr;  // mixed form: inner FP32 CG, outer residual
   sunhip::CGScal *h_sc = nullptr;   // pinned mirror
   sunhip::CGScal *h_poll = nullptr; // two pinned slots of pipelined convergence polling
+  unsigned long long *h_prog = nullptr; // pinned: the progress a solve's kernels report (solve tag, iteration, done)
+  unsigned prog_tag = 0;            // tag of the latest solve that reports there
   hipEvent_t evp[2] = {nullptr, nullptr};
   std::map<std::string, sunhip::Field> fields;
   std::map<std::string, float *> fields32;  // FP32 copies for the mixed form (cell layout)

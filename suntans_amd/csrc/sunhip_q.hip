@@ -688,9 +688,11 @@ int cg_iteration(sunhip_grid *g, const sunhip_cg_params *prm, QSolver<T> &S, int
 template <typename T>
 int cg_loop(sunhip_grid *g, const sunhip_cg_params *prm, QSolver<T> &S, int pk_apply, int pk_prec,
             bool finish = true) {
+  if (q_seg_ok(g, prm)) return q_seg_loop<T>(g, prm, S, pk_apply, pk_prec, finish);
+  int rc;
   int every = prm->check_every > 0 ? prm->check_every : (g->NT > (1 << 22) ? 4 : 8);
   if (every & 1) every++;
-  int it = 0, rc, slot = 0;
+  int it = 0, slot = 0;
   bool pending = false, done = false;
   // iterations enqueued after convergence return at once (device flag)
   while (!done && it < prm->maxiters) {
@@ -699,6 +701,23 @@ int cg_loop(sunhip_grid *g, const sunhip_cg_params *prm, QSolver<T> &S, int pk_a
     if ((rc = poll_chunk(g, S.sc, slot, pending, &done))) return rc;
   }
   if (finish) k_qfinish<T><<<nb4(g), 256, 0, g->stream>>>(g->geo(), S.x, S.p0, S.p1, S.sc);
+  HIPCHK(hipGetLastError());
+  return 0;
+}
+
+// The first application and fresh scalars of the iteration of
+// sunhip_qseg.hip.  Columns that are not computational keep p = src (see
+// k_qbnd_src), so where there are any the p buffers start from zero there too.
+template <typename T>
+int seg_start(sunhip_grid *g, const sunhip_cg_params *prm, QSolver<T> &S, const double *src, bool clear_x) {
+  const unsigned nf = (unsigned)((g->NT + 255) / 256);
+  if (g->has_bnd) {
+    k_fill<T><<<nf, 256, 0, g->stream>>>(S.p0, g->NT, T(0));
+    k_fill<T><<<nf, 256, 0, g->stream>>>(S.p1, g->NT, T(0));
+    if (clear_x) k_fill<T><<<nf, 256, 0, g->stream>>>(S.x, g->NT, T(0));
+  }
+  if (int rc = q_seg_start<T>(g, prm, S, clear_x)) return rc;
+  if (g->has_bnd && src) k_qbnd_src<<<nb4(g), 256, 0, g->stream>>>(g->geo(), src, reinterpret_cast<double *>(S.rtmp));
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -753,17 +772,26 @@ int qc_fcoef(sunhip_grid *g, double **out) {
 // caller put there: the reference reads a boundary neighbour's c as it
 // finds it), src /= c and q *= c on the computational columns, the scaled
 // coefficients, and OperatorQC in place of OperatorQ.
+// seg: for the iteration of sunhip_qseg.hip (the same values; the first sums
+// are left to its first kernel).
 int q_setup(sunhip_grid *g, const sunhip_cg_params *prm, F64 &B, QSolver<double> &S, CGScal *stage = nullptr,
-            CGScal *sc = nullptr) {
+            CGScal *sc = nullptr, bool seg = false) {
   int rc = check_q(g, prm);
   if (rc) return rc;
   if ((rc = f64bufs(g, B))) return rc;
   S = solver64(g, B);
   if (sc) S.sc = sc;
-  if ((rc = upload_scal(g, S.sc, prm, stage))) return rc;
   const Geo G = g->geo();
   QVec<double, double> V{};
   V.coef = B.coef->d; V.dzf = B.dzf->d; V.D = B.D->d; V.vin = B.q->d; V.src = B.src->d; V.out = B.r->d;
+  if (seg) {
+    Field *ql;
+    if ((rc = field(g, "qlp", &ql))) return rc;
+    S.ql = ql->d;
+    if ((rc = q_seg_setup64(g, B.dzz->d, B.coef->d, B.bq->d, S.ql)) || (rc = q_seg_resid64(g, V))) return rc;
+    return seg_start<double>(g, prm, S, B.src->d, false);
+  }
+  if ((rc = upload_scal(g, S.sc, prm, stage))) return rc;
   if (prm->precond == 1) {
     Field *c;
     double *fc;
@@ -806,8 +834,9 @@ int q_unscale(sunhip_grid *g, const sunhip_cg_params *prm, const F64 &B) {
   return 0;
 }
 
+// d null: the scalars are on their way to g->h_sc already.
 int q_stats(sunhip_grid *g, CGScal *d, sunhip_cg_stats *st) {
-  HIPCHK(hipMemcpyAsync(g->h_sc, d, sizeof(CGScal), hipMemcpyDeviceToHost, g->stream));
+  if (d) HIPCHK(hipMemcpyAsync(g->h_sc, d, sizeof(CGScal), hipMemcpyDeviceToHost, g->stream));
   HIPCHK(hipEventRecord(g->ev2, g->stream));
   HIPCHK(hipStreamSynchronize(g->stream));
   if (st) {
@@ -873,7 +902,8 @@ int q_end32(sunhip_grid *g, const QSolver<float> &S) {
   return 0;
 }
 
-int q_mixed_prepare(sunhip_grid *g, const sunhip_cg_params *prm, QSolver<float> *S32, QVec<double, float> *R) {
+int q_mixed_prepare(sunhip_grid *g, const sunhip_cg_params *prm, QSolver<float> *S32, QVec<double, float> *R,
+                    bool seg) {
   HIPCHK(hipSetDevice(g->device));
   int rc = check_q(g, prm);
   if (rc) return rc;
@@ -892,10 +922,16 @@ int q_mixed_prepare(sunhip_grid *g, const sunhip_cg_params *prm, QSolver<float> 
   k_cast<double, float><<<(unsigned)((g->NE + 255) / 256), 256, 0, g->stream>>>(B.dzf->d, f32, g->NE);
   k_cast<double, float><<<(unsigned)((g->NES + 255) / 256), 256, 0, g->stream>>>(B.D->d, g->d_D32, g->NES);
   HIPCHK(hipGetLastError());
-  if ((rc = launch_factor<float>(g, c32, b32))) return rc;
   ZReg Z{};
-  if ((rc = q_windows(g, B.coef->d, B.dzf->d, &Z))) return rc;
+  float *l32 = nullptr;
+  if (seg) {  // the iteration of sunhip_qseg.hip reads the coefficients
+    if ((rc = field32(g, "ql", &l32)) || (rc = q_seg_factor32(g, c32, b32, l32))) return rc;
+  } else {
+    if ((rc = launch_factor<float>(g, c32, b32))) return rc;
+    if ((rc = q_windows(g, B.coef->d, B.dzf->d, &Z))) return rc;
+  }
   *S32 = QSolver<float>{g->d_ms, c32, f32, g->d_D32, x32, r32, z32, t32, pa, pb, b32};
+  S32->ql = l32;
   S32->Z = Z;
   QVec<double, float> V{};
   V.coef = B.coef->d; V.dzf = B.dzf->d; V.D = B.D->d; V.vin = B.q->d; V.src = B.src->d; V.out = r32;
@@ -968,11 +1004,13 @@ int sunhip_q_solve(sunhip_grid *g, const sunhip_cg_params *prm, sunhip_cg_stats 
   QSolver<double> S;
   int rc;
   HIPCHK(hipEventRecord(g->ev0, g->stream));
-  if ((rc = q_setup(g, prm, B, S))) return rc;
+  read_tuning(g);
+  const bool seg = q_seg_ok(g, prm);
+  if ((rc = q_setup(g, prm, B, S, nullptr, nullptr, seg))) return rc;
   HIPCHK(hipEventRecord(g->ev1, g->stream));
   if ((rc = cg_loop<double>(g, prm, S, PK_QAPPLY, PK_QPREC))) return rc;
   if ((rc = q_unscale(g, prm, B))) return rc;
-  return q_stats(g, g->d_qs, st);
+  return q_stats(g, seg ? nullptr : g->d_qs, st);
 }
 
 int sunhip_q_solve_fixed(sunhip_grid *g, const sunhip_cg_params *prm, int n, sunhip_cg_stats *st) {
@@ -984,14 +1022,13 @@ int sunhip_q_solve_fixed(sunhip_grid *g, const sunhip_cg_params *prm, int n, sun
   QSolver<double> S;
   int rc;
   HIPCHK(hipEventRecord(g->ev0, g->stream));
-  if ((rc = q_setup(g, &p, B, S))) return rc;
+  read_tuning(g);
+  const bool seg = q_seg_ok(g, &p);
+  if ((rc = q_setup(g, &p, B, S, nullptr, nullptr, seg))) return rc;
   HIPCHK(hipEventRecord(g->ev1, g->stream));
-  for (int it = 0; it < n; it++)
-    if ((rc = cg_iteration<double>(g, &p, S, it, PK_QAPPLY, PK_QPREC))) return rc;
-  k_qfinish<double><<<nb4(g), 256, 0, g->stream>>>(g->geo(), S.x, S.p0, S.p1, S.sc);
-  HIPCHK(hipGetLastError());
+  if ((rc = cg_loop<double>(g, &p, S, PK_QAPPLY, PK_QPREC))) return rc;
   if ((rc = q_unscale(g, &p, B))) return rc;
-  return q_stats(g, g->d_qs, st);
+  return q_stats(g, seg ? nullptr : g->d_qs, st);
 }
 
 // Mixed precision (FP32 inner PCG inside FP64 iterative refinement):
@@ -1005,7 +1042,9 @@ int sunhip_q_solve_mixed(sunhip_grid *g, const sunhip_cg_params *prm, double inn
   HIPCHK(hipEventRecord(g->ev0, g->stream));
   QSolver<float> S;
   QVec<double, float> R;
-  int rc = q_mixed_prepare(g, prm, &S, &R);
+  read_tuning(g);
+  const bool seg = q_seg_ok(g, prm);
+  int rc = q_mixed_prepare(g, prm, &S, &R, seg);
   if (rc) return rc;
   CGScal *so = g->d_mo;
   sunhip_cg_params inner = *prm;
@@ -1032,13 +1071,14 @@ int sunhip_q_solve_mixed(sunhip_grid *g, const sunhip_cg_params *prm, double inn
     // inner FP32 PCG from e = 0, asked for no more reduction than the outer
     // target still needs (with a margin for the FP32/FP64 residual gap)
     inner.epsilon = std::max(inner_tol, 0.25 * prm->epsilon / ratio);
-    if ((rc = q_inner_begin(g, &inner, S, nullptr))) return rc;
+    if ((rc = seg ? seg_start<float>(g, &inner, S, nullptr, true) : q_inner_begin(g, &inner, S, nullptr))) return rc;
     if ((rc = cg_loop<float>(g, &inner, S, PK_MAPPLY, PK_MPREC, false))) return rc;
+    const CGScal *sc = seg ? S.sc + 1 : S.sc;  // the settled scalars
     // x += e (with the inner solve's last update), the next residual, then
     // one wait for both the inner count and the residual
-    k_mix_finish<<<nb4(g), 256, 0, g->stream>>>(g->geo(), const_cast<double *>(R.vin), S.x, S.p0, S.p1, S.sc);
+    k_mix_finish<<<nb4(g), 256, 0, g->stream>>>(g->geo(), const_cast<double *>(R.vin), S.x, S.p0, S.p1, sc);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(&g->h_poll[0], S.sc, sizeof(CGScal), hipMemcpyDeviceToHost, g->stream));
+    HIPCHK(hipMemcpyAsync(&g->h_poll[0], sc, sizeof(CGScal), hipMemcpyDeviceToHost, g->stream));
     if ((rc = residual())) return rc;
     HIPCHK(hipStreamSynchronize(g->stream));
     total_inner += g->h_poll[0].iter;

@@ -173,9 +173,13 @@ __device__ __forceinline__ void qfactor_tile(const Geo &G, const T *__restrict__
                                              int l) {
   if (t >= G.Nt) return;
   const int s = t * 64 + l, n = G.nk[s], kt = G.ctop[s];
-  if (n == 0 || G.comp[s] != 1 || kt >= n - 1) return;
+  if (n == 0 || G.comp[s] != 1) return;
   const int64_t base = G.toff[t] + l;
   T lprev = 0;
+  if (kt >= n - 1) {  // one layer: u = -r/(2 coef) (main/phys.c:3603-3604)
+    if (kt == n - 1) bq[base + (int64_t)kt * 64] = T(-0.5) / coef[base + (int64_t)kt * 64];
+    return;
+  }
   T ck = coef[base + (int64_t)kt * 64];
   for (int k = kt; k < n; k++) {
     const int64_t idx = base + (int64_t)k * 64;
@@ -984,7 +988,7 @@ __device__ __forceinline__ void qprec_tile(const Geo &G, const T *__restrict__ c
     const uint32_t idx = base + (uint32_t)kt * 64u;
     T rk = at32(r, idx);
     if (UPDATE) { rk = rk - nu * at32(z, idx); at32(r, idx) = rk; }
-    const T u = T(-0.5) * rk / C(kt);
+    const T u = rk * (T(-0.5) / C(kt));
     at32(out, idx) = u;
     rz += (double)rk * (double)u;
     rr += (double)rk * (double)rk;

@@ -18,6 +18,7 @@ struct QSolver {
   T *x, *r, *z, *rtmp, *p0, *p1, *bq;
   const T *fcoef;  // qprecond=1: the scaled face coefficients
   ZReg Z;          // z-level windows of this solve (cwin null: none)
+  T *ql;           // the rows' l (the iteration of sunhip_qseg.hip)
 };
 
 // One free-surface PCG instance.
@@ -36,6 +37,29 @@ int set_zdz(sunhip_grid *g, const double *dz);
 // off ("zreg" 0).
 int q_windows(sunhip_grid *g, const double *coef, const double *dzf, ZReg *Z);
 
+// The iteration of small and middle grids (sunhip_qseg.hip): one block per
+// tile.  At most SUNHIP_QSEG_TILES tiles, the defaults of the other kernels'
+// knobs, and qprecond=2.  Per iteration, these kernels against the
+// one-lane-per-column ones and their finishers: 32 tiles of 50 levels 27 / 69
+// us, 220 tiles of hexagons 33 / 87, 381 tiles 38 / 71, 817 tiles of 61 levels
+// 69 / 106, 790 tiles of 80 levels 87 / 117; at 1570 tiles of 80 levels 190 /
+// 135, every CU then having waves enough either way.
+#define SUNHIP_QSEG_TILES 1024
+bool q_seg_ok(const sunhip_grid *g, const sunhip_cg_params *prm);
+// Coefficients, inverse pivots and l (QSolver::ql) from dzz, or the last two
+// from FP32 coefficients.
+int q_seg_setup64(sunhip_grid *g, const double *dzz, double *coef, double *bq, double *ql);
+int q_seg_factor32(sunhip_grid *g, float *coef, float *bq, float *ql);
+// V.out = V.src - L V.vin
+int q_seg_resid64(sunhip_grid *g, const QVec<double, double> &V);
+// rtmp = M^-1 r, p0 = 0 (and x = 0), fresh scalars with their first step pending.
+template <typename T>
+int q_seg_start(sunhip_grid *g, const sunhip_cg_params *prm, QSolver<T> &S, bool clear_x);
+// Iterate until the device says done; the scalars then are in g->h_sc (after a
+// wait for the stream) and at S.sc + 1, and (finish) x has its last update.
+template <typename T>
+int q_seg_loop(sunhip_grid *g, const sunhip_cg_params *prm, QSolver<T> &S, int pk_apply, int pk_prec, bool finish);
+
 // Upload fresh CG scalars (tolerance, limits) to d from the pinned host slot
 // stage (g->h_sc when null).  The slot must not be rewritten before the
 // stream has executed the copy.
@@ -50,8 +74,10 @@ int q_end32(sunhip_grid *g, const QSolver<float> &S);
 
 // Mixed form: FP64 coefficients, FP32 copies of coef/dzf/D, FP32 pivots;
 // S32 gets the FP32 PCG buffers (x = the correction e, scalars g->d_ms) and
-// R the FP64 residual operands (out = the FP32 residual).
-int q_mixed_prepare(sunhip_grid *g, const sunhip_cg_params *prm, QSolver<float> *S32, QVec<double, float> *R);
+// R the FP64 residual operands (out = the FP32 residual).  seg: for the
+// iteration of sunhip_qseg.hip.
+int q_mixed_prepare(sunhip_grid *g, const sunhip_cg_params *prm, QSolver<float> *S32, QVec<double, float> *R,
+                    bool seg = false);
 // Inner FP32 PCG from e = 0 on the residual already in S32.r.
 int q_inner_begin(sunhip_grid *g, const sunhip_cg_params *inner, QSolver<float> &S32, CGScal *stage);
 // x64 += e32.

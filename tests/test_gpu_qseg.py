@@ -1,0 +1,70 @@
+"""The pressure solve's iteration on small and middle grids (one block per
+tile, one wave per eight levels) against the one-lane-per-column kernels: the
+same values, sums and iteration counts, bit for bit.  Grids at the edges of
+tiles, groups of four tiles, segments of eight levels and waves of one or
+two segments, of every face class, with one-layer columns, surfaces that cross
+layers and boundary columns that are not computational."""
+import numpy as np
+import pytest
+
+from suntans_amd import cases, device
+
+pytestmark = pytest.mark.gpu
+
+# (cells per row, rows, levels): 64 cells per tile, 4 tiles per group
+SIZES = [(2, 3, 8), (8, 4, 7), (31, 1, 9), (32, 1, 16), (16, 8, 17), (33, 4, 24), (40, 13, 63), (16, 9, 64), (16, 9, 65),
+         (23, 11, 100), (9, 7, 127), (9, 7, 128), (64, 66, 12)]
+
+
+def solve(st, mixed, tuning=(), fixed=None):
+    dg = device.DeviceGrid(st)
+    device.member_upload(dg, st)
+    for k, v in tuning:
+        dg.tune(k, v)
+    if mixed:
+        s = dg.q_solve_mixed(epsilon=1e-10, inner_tol=1e-4)
+        n = (s["niters"], s["inner_iters"])
+    else:
+        s = dg.q_solve(epsilon=1e-10, fixed=fixed)
+        n = s["niters"]
+    q = dg.download("q", dg.sizes()["Nflat"])
+    s2 = dg.q_solve(epsilon=1e-10)  # once more from the solution, on used buffers
+    q2 = dg.download("q", dg.sizes()["Nflat"])
+    dg.close()
+    return q, n, q2, s["resid"]
+
+
+def same(st, mixed=False, fixed=None):
+    a = solve(st, mixed, (), fixed)
+    b = solve(st, mixed, [("prec_unroll", 4)], fixed)
+    assert a[1] == b[1] and a[3] == b[3]
+    assert np.array_equal(a[0], b[0]) and np.array_equal(a[2], b[2])
+
+
+@pytest.mark.parametrize("nx,ny,levels", SIZES, ids=["%dx%dx%d" % s for s in SIZES])
+def test_sizes(gpu_available, nx, ny, levels):
+    st = cases.tiny(nx + levels, nx=nx, ny=max(ny, 1), Nkmax=levels, min_layers=min(3, levels - 4))
+    same(st)
+    same(st, mixed=True)
+
+
+@pytest.mark.parametrize("fixed", [1, 2, 3])
+def test_fixed_iterations(gpu_available, fixed):
+    same(cases.lock_exchange(seed=3), fixed=fixed)
+
+
+SHAPES = {
+    "quad": dict(planform="quad", nx=19, ny=13, Nkmax=21),
+    "quadtri": dict(planform="quad", split_every=3, nx=19, ny=13, Nkmax=70),
+    "hex": dict(planform="hex", nx=13, ny=9, Nkmax=15),
+    "hex8": dict(planform="hex", split_every=4, maxfaces=7, nx=13, ny=9, Nkmax=40),
+    "open": dict(nx=17, ny=11, Nkmax=20, open_marks=cases.open_ends()),
+    "onelayer": dict(nx=17, ny=11, Nkmax=4, min_layers=0),
+}
+
+
+@pytest.mark.parametrize("name", sorted(SHAPES))
+def test_shapes(gpu_available, name):
+    st = cases.tiny(5, **SHAPES[name])
+    same(st)
+    same(st, mixed=True)
