@@ -224,7 +224,7 @@ struct sunhip_grid {
                          // 2 on with a 4-waves-per-SIMD register budget, 3 on with 2 levels per group,
                          // -1 (default) 2 from 4096 tiles up, off below (short walks favour the plain kernel)
   int tune_phead = -1;   // top levels per column the preconditioner keeps in registers (0, 8, 16, 24, 32);
-                         // -1 (default) QHead's from 1024 tiles up in FP64, 2048 in FP32, 0 below
+                         // -1 (default) QHead's from 1024 tiles up, 0 below
   int tune_band = 0;     // operator kernel over level bands of this many levels (0: whole columns)
 
   // per-kernel timing (sunhip_profile): an event pair around every launch of

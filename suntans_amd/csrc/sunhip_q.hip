@@ -193,7 +193,7 @@ __global__ __launch_bounds__(256, MINW > 0 ? MINW : 1) void k_qapply_xp(Geo G, Q
 }
 
 // Vertical-line preconditioner (qprec_tile) over all tiles, 4 per block.
-template <bool UPDATE, int U, typename T, bool RZID = false, int KR = 0, bool ZR = false, int KL = 0>
+template <bool UPDATE, int U, typename T, bool RZID = false, int KR = 0, bool ZR = false, int KL = 0, bool NT = true>
 __global__ __launch_bounds__(256) void k_qprec(Geo G, const T *__restrict__ coef, const T *__restrict__ z,
                                                T *__restrict__ r, T *__restrict__ out, const T *__restrict__ bq,
                                                CGScal *sc, Red R, ZReg Z) {
@@ -203,10 +203,10 @@ __global__ __launch_bounds__(256) void k_qprec(Geo G, const T *__restrict__ coef
   const int t = tile_group(G, blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6);
   double rz = 0, rr = 0;
   if (ZR && t < G.Nt && Z.tflag[t])
-    qprec_tile<UPDATE, U, T, RZID, KR, true, KL>(G, coef, z, r, out, bq, UPDATE ? (T)sc->nu : T(0), t,
+    qprec_tile<UPDATE, U, T, RZID, KR, true, KL, NT>(G, coef, z, r, out, bq, UPDATE ? (T)sc->nu : T(0), t,
                                                  threadIdx.x & 63, rz, rr, &Z, lrows + threadIdx.x);
   else
-    qprec_tile<UPDATE, U, T, RZID, KR, false, KL>(G, coef, z, r, out, bq, UPDATE ? (T)sc->nu : T(0), t,
+    qprec_tile<UPDATE, U, T, RZID, KR, false, KL, NT>(G, coef, z, r, out, bq, UPDATE ? (T)sc->nu : T(0), t,
                                                   threadIdx.x & 63, rz, rr, &Z, lrows + threadIdx.x);
   double v[2] = {rz, rr};
   reduce_out<2, 256>(v, R, sc);
@@ -439,10 +439,10 @@ int launch_prec(sunhip_grid *g, CGScal *sc, const T *coef, const T *z, T *r, T *
   // unknowns heads of 24, 32, 40 and 48 levels with 16 in LDS take 460, 421,
   // 390 and 467 us in FP64 (40: 2 waves per SIMD, 48 spills) and 231, 212,
   // 219 and 207 us in FP32; without the LDS stage 32 levels take 485 and
-  // 248 us.  Few tiles (below 1024 in FP64, 2048 in FP32) take the plain
-  // sweep.
+  // 248 us.  Few tiles (below 1024) take the plain sweep.
   const bool fp32 = std::is_same<T, float>::value;
-  const int head = g->tune_phead >= 0 ? g->tune_phead : (g->Nt >= (fp32 ? 2048 : 1024) ? 40 : 0);
+  const bool nt = g->NT * (int64_t)sizeof(T) >= SUNHIP_STREAM_BYTES;
+  const int head = g->tune_phead >= 0 ? g->tune_phead : (g->Nt >= 1024 ? 40 : 0);
   if constexpr (!UPDATE) {
     PREC(4, 0);  // once per solve; every variant gives the same bits
   } else if (head == 0) {
@@ -464,7 +464,18 @@ int launch_prec(sunhip_grid *g, CGScal *sc, const T *coef, const T *z, T *r, T *
         else PREC(4, 24);
         break;
       case 32: PREC(4, 32); break;
-      default: PREC3(4, QHead<T>::regs, QHead<T>::lds); break;
+      default:
+        if (rzid && !nt) {  // the vectors stay in the memory-side cache (see launch_apply)
+          if (zr)
+            k_qprec<UPDATE, 4, T, true, QHead<T>::regs, true, QHead<T>::lds, false>
+                <<<nb, 256, 0, g->stream>>>(G, coef, z, r, out, bq, sc, R, ZZ);
+          else
+            k_qprec<UPDATE, 4, T, true, QHead<T>::regs, false, QHead<T>::lds, false>
+                <<<nb, 256, 0, g->stream>>>(G, coef, z, r, out, bq, sc, R, ZZ);
+        } else {
+          PREC3(4, QHead<T>::regs, QHead<T>::lds);
+        }
+        break;
     }
   }
 #undef PREC
@@ -480,7 +491,15 @@ template <int MODE, typename T, typename TO>
 int launch_apply(sunhip_grid *g, CGScal *sc, const QVec<T, TO> &V, const Red &R, int pk = -1) {
   // launch-shape variants (tiles per block, streaming stores) exist for the
   // fused iteration kernel on triangles at the default unroll
-  const bool variants = MODE == QM_FUSED && g->mf <= 3 && g->tune_unroll == 4;
+  // (with no other shape asked for, small launches take the plain kernel below)
+  const bool dflt = g->tune_unroll == 4 && g->tune_xchg < 0 && g->tune_tiles == 4 && !g->tune_blk && !g->tune_band &&
+                    !g->tune_minw && g->tune_nts;
+  const bool variants = MODE == QM_FUSED && g->mf <= 3 && g->tune_unroll == 4 && !dflt;
+  // streaming stores pay once the iteration's vectors overflow the 256 MB
+  // memory-side cache: 3900 tiles (1.3e7 unknowns) 204 us against 210, but
+  // 1570 tiles (2.1e6) 81 against 80 with the preconditioner after it at 50
+  // against 39
+  const bool nts = g->tune_nts && g->NT * (int64_t)sizeof(T) >= SUNHIP_STREAM_BYTES;
   const int tpb = variants ? g->tune_tiles : 4;
   const int nba = (g->Nt + tpb - 1) / tpb;
   const Geo G = g->geo();
@@ -495,8 +514,15 @@ int launch_apply(sunhip_grid *g, CGScal *sc, const QVec<T, TO> &V, const Red &R,
 #define APPLYV(TPB, NTS) k_qapply<MODE, 3, 4, T, TO, TPB, NTS><<<nba, TPB * 64, 0, g->stream>>>(G, V, sc, R)
 #define APPLYW(NTS, W) k_qapply<MODE, 3, 4, T, TO, 4, NTS, W><<<nba, 256, 0, g->stream>>>(G, V, sc, R)
   if constexpr (MODE == QM_FUSED && std::is_same<T, TO>::value) {
-    // the exchange kernel, unless another launch shape was asked for
-    const int xmode = g->tune_xchg >= 0 ? g->tune_xchg : (g->Nt >= 4096 ? 2 : 0);
+    // The exchange kernel, unless another launch shape was asked for.  With
+    // few tiles the plain kernel at 2 levels per group has more waves in
+    // flight: 790 tiles of triangles 50 us against 58 (q50k), 1570 tiles 83
+    // against 80, 3900 tiles 239 against 204; with 6 or 8 faces the exchange
+    // saves most gathers at any size (1090 tiles of hexagons 114 against 86).
+    // Its register budget of 4 waves per SIMD spills from 4 faces up (780
+    // tiles of quadrilaterals 93 us against 54 without the budget).
+    const bool few = g->Nt < 1536 && g->mf <= 4;
+    const int xmode = g->tune_xchg >= 0 ? g->tune_xchg : (few ? 0 : g->mf <= 3 ? 2 : 1);
     if (zr && xmode >= 4 && g->max_pairs <= SUNHIP_XPAIRS && g->tune_unroll == 4) {
       // the pipelined exchange kernel: 4 two-level groups (xchg 4), 4 four-level
       // groups under a 4-wave register budget (5), or 2 two-level groups at
@@ -536,11 +562,11 @@ int launch_apply(sunhip_grid *g, CGScal *sc, const QVec<T, TO> &V, const Red &R,
     else k_qapply_x<NF, U, T, NTS, W><<<nbx, 256, 0, g->stream>>>(G, V, sc, R);                 \
   } while (0)
         if (xmode == 2) {  // register budget of 4 waves per SIMD
-          if (g->tune_nts) XCH(UX, true, 4); else XCH(UX, false, 4);
+          if (nts) XCH(UX, true, 4); else XCH(UX, false, 4);
         } else if (xmode == 3) {  // 2 levels per group
-          if (g->tune_nts) XCH(2, true, 0); else XCH(2, false, 0);
+          if (nts) XCH(2, true, 0); else XCH(2, false, 0);
         } else {
-          if (g->tune_nts) XCH(UX, true, 0); else XCH(UX, false, 0);
+          if (nts) XCH(UX, true, 0); else XCH(UX, false, 0);
         }
 #undef XCH
         return 0;
@@ -585,10 +611,11 @@ int launch_apply(sunhip_grid *g, CGScal *sc, const QVec<T, TO> &V, const Red &R,
     else if (tpb == 16) { if (g->tune_nts) APPLYV(16, true); else APPLYV(16, false); }
     else APPLYV(4, true);
   } else if (g->mf <= 3) {
-    if (g->tune_unroll == 1) APPLY(3, 1); else if (g->tune_unroll == 2) APPLY(3, 2);
+    if (g->tune_unroll == 1) APPLY(3, 1); else if (g->tune_unroll == 2 || (dflt && MODE == QM_FUSED)) APPLY(3, 2);
     else if (g->tune_unroll == 8) APPLY(3, 8); else APPLY(3, 4);
   } else if (g->mf == 4) {
-    if (g->tune_unroll == 1) APPLY(4, 1); else if (g->tune_unroll == 2) APPLY(4, 2); else APPLY(4, 4);
+    if (g->tune_unroll == 1) APPLY(4, 1); else if (g->tune_unroll == 2 || (dflt && MODE == QM_FUSED)) APPLY(4, 2);
+    else APPLY(4, 4);
   } else if (g->mf <= 6) {  // 2 levels per group at most: 6 or 8 gathers per level
     if (g->tune_unroll == 1) APPLY(6, 1); else APPLY(6, 2);
   } else {

@@ -969,7 +969,8 @@ template <typename T>
 struct QHead {
   static constexpr int regs = sizeof(T) == 8 ? 40 : 48, lds = 16;
 };
-template <bool UPDATE, int U, typename T, bool RZID = false, int KR = 0, bool ZR = false, int KL = 0>
+// NT: r and out stored with the non-temporal hint.
+template <bool UPDATE, int U, typename T, bool RZID = false, int KR = 0, bool ZR = false, int KL = 0, bool NT = true>
 __device__ __forceinline__ void qprec_tile(const Geo &G, const T *__restrict__ coef, const T *__restrict__ z,
                                            T *__restrict__ r, T *__restrict__ out, const T *__restrict__ bq, T nu,
                                            int t, int l, double &rz, double &rr, const ZReg *Zp = nullptr,
@@ -999,7 +1000,7 @@ __device__ __forceinline__ void qprec_tile(const Geo &G, const T *__restrict__ c
   // e and l out
   auto row = [&](int k, T rv, T zv, T ck, T cn, T &e, T &lk) -> T {
     T rk = rv;
-    if (UPDATE) { rk = rk - nu * zv; st_stream<true>(&at32(r, base + (uint32_t)k * 64u), rk); }
+    if (UPDATE) { rk = rk - nu * zv; st_stream<NT>(&at32(r, base + (uint32_t)k * 64u), rk); }
     sr.add(k, (double)rk * (double)rk);
     const T ck1 = k == n - 1 ? T(0) : cn;
     const T ib = q_pivot<T>(k, kt, n, ck, ck1, lprev);
@@ -1092,7 +1093,7 @@ __device__ __forceinline__ void qprec_tile(const Geo &G, const T *__restrict__ c
       const int k = ke - j;
       if (k >= klo) {
         const T u = ev[j] - (cv[j] * iv[j]) * unext;
-        st_stream<true>(&at32(out, base + (uint32_t)k * 64u), u);
+        st_stream<NT>(&at32(out, base + (uint32_t)k * 64u), u);
         if constexpr (!RZID) uz += (double)rv[j] * (double)u;
         unext = u;
       }
@@ -1103,7 +1104,7 @@ __device__ __forceinline__ void qprec_tile(const Geo &G, const T *__restrict__ c
       const T *w = lrow + (2 * (k - kls)) * 256;
       const T u = w[0] - w[256] * unext;
       const uint32_t idx = base + (uint32_t)k * 64u;
-      st_stream<true>(&at32(out, idx), u);
+      st_stream<NT>(&at32(out, idx), u);
       if constexpr (!RZID) uz += (double)at32((const T *)r, idx) * (double)u;
       unext = u;
     }
@@ -1114,7 +1115,7 @@ __device__ __forceinline__ void qprec_tile(const Geo &G, const T *__restrict__ c
       const int k = kt + j;
       if (k < n) {
         const T u = he[j] - hl[j] * unext;
-        st_stream<true>(&at32(out, base + (uint32_t)k * 64u), u);
+        st_stream<NT>(&at32(out, base + (uint32_t)k * 64u), u);
         if constexpr (!RZID) uz += (double)hr[j] * (double)u;
         unext = u;
       }

@@ -10,6 +10,10 @@
 
 namespace sunhip {
 
+// Bytes of a cell field from which the iteration's seven vectors overflow the
+// 256 MB memory-side cache, so that a launch's results are streamed.
+#define SUNHIP_STREAM_BYTES (64 << 20)
+
 // One pressure PCG instance: storage type, its scalars and its buffers.
 template <typename T>
 struct QSolver {

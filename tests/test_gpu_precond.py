@@ -42,3 +42,27 @@ def test_head_against_plain_sweep(gpu_available, levels):
     # both stop at a true residual of 1e-10
     assert s2["converged"]
     assert np.linalg.norm(q2 - q0) <= 1e-8 * np.linalg.norm(q0)
+
+
+@pytest.mark.parametrize("kw", [dict(nx=190, ny=180, Nkmax=6), dict(planform="quad", nx=270, ny=250, Nkmax=6),
+                                dict(planform="hex", nx=270, ny=250, Nkmax=6)], ids=["tri", "quad", "hex"])
+def test_default_kernels_above_1024_tiles(gpu_available, kw):
+    """The kernels a solve of a little over 1024 tiles takes by default
+    (cached stores, register head, the plain or the exchange operator)
+    against the plain ones, bit for bit."""
+    st = cases.tiny(9, **kw)
+    assert (st.Nc + 63) // 64 > 1024
+    out = []
+    for tuning in ((), (("xchg", 0), ("unroll", 1), ("prec_head", 0))):
+        dg = device.DeviceGrid(st)
+        device.member_upload(dg, st)
+        for k, v in tuning:
+            dg.tune(k, v)
+        n = dg.q_solve(epsilon=1e-10)["niters"]
+        out.append((n, dg.download("q", dg.sizes()["Nflat"])))
+        dg.upload("q", st.get("qc"))
+        n = dg.q_solve_mixed(epsilon=1e-10, inner_tol=1e-4)["inner_iters"]
+        out[-1] += (n, dg.download("q", dg.sizes()["Nflat"]))
+        dg.close()
+    assert out[0][0] == out[1][0] and out[0][2] == out[1][2]
+    assert np.array_equal(out[0][1], out[1][1]) and np.array_equal(out[0][3], out[1][3])
