@@ -256,6 +256,22 @@ enum { PK_QAPPLY = 0, PK_QPREC = 1, PK_HAPPLY = 2, PK_HPREC = 3, PK_MAPPLY = 4, 
 }  // namespace sunhip
 
 namespace sunhip {
+// The levels of a launch's tiles in nb bands of len levels, one wave per tile
+// and band, for kernels whose levels do not depend on each other: with few
+// tiles one wave per tile would leave most of the chip idle.  Bands of 8
+// levels or more, and no more of them than fill the chip (4096 waves).
+struct Bands {
+  int nb, len;
+};
+inline Bands level_bands(const sunhip_grid *g, int tiles) {
+  const int most = (g->maxdepth + 1 + 7) / 8;  // w-type levels too
+  int nb = tiles > 0 ? (4096 + tiles - 1) / tiles : 1;
+  nb = nb < 1 ? 1 : nb > most ? most : nb;
+  if (nb <= 1) return Bands{1, 0x3fffffff};
+  const int len = ((g->maxdepth + 1 + nb - 1) / nb + 7) / 8 * 8;
+  return Bands{(g->maxdepth + 1 + len - 1) / len, len};
+}
+
 int field(sunhip_grid *g, const char *name, Field **out);  // create on demand
 int field32(sunhip_grid *g, const char *name, float **out);
 Kind kind_of(const char *name);

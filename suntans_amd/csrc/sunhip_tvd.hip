@@ -23,13 +23,44 @@
 using namespace sunhip;
 
 
-template <int NF, int GRP>
-__global__ __launch_bounds__(256) void k_tvd_sums(Geo G, TvdArgs A) {
-  tvd_sums_tile<NF, GRP>(G, A, xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), threadIdx.x & 63);
+// BAND: the tiles' levels in bands (Bands), one wave per tile and band; else
+// one wave per tile.
+template <int NF, int GRP, bool BAND = false>
+__global__ __launch_bounds__(256) void k_tvd_sums(Geo G, TvdArgs A, Bands B = {}) {
+  const int v = xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
+  if (!BAND) { tvd_sums_tile<NF, GRP>(G, A, v, l); return; }
+  const int t = v / B.nb, k0 = (v - t * B.nb) * B.len;
+  tvd_sums_tile<NF, GRP>(G, A, t, l, k0, k0 + B.len);
 }
 
-__global__ __launch_bounds__(256) void k_tvd_faces(Geo G, TvdArgs A) {
-  tvd_faces_tile(G, A, xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), threadIdx.x & 63);
+template <bool BAND>
+__global__ __launch_bounds__(256) void k_tvd_faces(Geo G, TvdArgs A, Bands B) {
+  const int v = xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
+  if (!BAND) { tvd_faces_tile(G, A, v, l); return; }
+  const int t = v / B.nb, k0 = (v - t * B.nb) * B.len;
+  tvd_faces_tile(G, A, t, l, k0, k0 + B.len);
+}
+
+// The column update by segments (update_column_seg), one block per tile.  A
+// lane that walks a whole column waits out each level's loads and nine
+// divisions in turn (50 levels: 97 us on any grid); with a wave per 8 levels
+// only the elimination is serial.  The rows take 214 VGPRs and up, one block
+// per CU, so it pays while there are few blocks per CU: 129 tiles of 37 levels
+// 78 -> 34 us, 500 of 50 103 -> 71, 820 of 61 levels 131 -> 132; with 16 levels
+// per wave (more than 64 levels) 75 tiles of 100 levels 193 -> 76 us, 240 of
+// 90 176 -> 75, but spills cost more than it gives from 6 faces (280 tiles
+// of 67 levels 141 -> 155).  First-order upwind (pre false) gathers its fluxes
+// here and spills from 6 faces too; 129 tiles of quadrilaterals 65 -> 40 us.
+template <int NF>
+static bool tvd_seg(const sunhip_grid *g, bool pre) {
+  if (g->tune_tvdgrp != 2 || g->tune_tvdhead != 8 || (!pre && NF > 4)) return false;
+  return g->maxdepth <= 8 * SUNHIP_SEG ? g->Nt <= 768 : NF <= 4 && g->maxdepth <= 16 * SUNHIP_SEG && g->Nt <= 512;
+}
+template <int NF, bool PRE, int SPW>
+__global__ __launch_bounds__(512, 2) void k_update_column_seg(Geo G, ColArgs A) {
+  __shared__ double pass[4][64];
+  const int t = xcd_block(blockIdx.x, gridDim.x);
+  update_column_seg<NF, PRE, SPW>(G, A, t, pass);
 }
 
 template <int NF, int GRP, bool SRC = false, bool PRE = false, int KR = 0>
@@ -87,15 +118,20 @@ int face_scalars_launch(sunhip_grid *g, const TvdArgs &A) {
   int ps = prof_begin(g, PK_TSUMS);
   with_nf(g->mf, [&](auto nf) {
     constexpr int NF = decltype(nf)::value;
-    const unsigned nb = (unsigned)((g->Nt + 3) / 4);
-    if (g->tune_sumsgrp == 4) k_tvd_sums<NF, 4><<<nb, 256, 0, g->stream>>>(G, A);
+    const Bands B = level_bands(g, g->Nt);
+    const unsigned nb = (unsigned)((g->Nt + 3) / 4), nbb = (unsigned)(((int64_t)g->Nt * B.nb + 3) / 4);
+    if (g->tune_sumsgrp == 4 && B.nb > 1) k_tvd_sums<NF, 4, true><<<nbb, 256, 0, g->stream>>>(G, A, B);
+    else if (g->tune_sumsgrp == 4) k_tvd_sums<NF, 4><<<nb, 256, 0, g->stream>>>(G, A);
     else if (g->tune_sumsgrp == 2) k_tvd_sums<NF, 2><<<nb, 256, 0, g->stream>>>(G, A);
     else k_tvd_sums<NF, 1><<<nb, 256, 0, g->stream>>>(G, A);
     return 0;
   });
   prof_end(g, ps);
   ps = prof_begin(g, PK_TFACES);
-  k_tvd_faces<<<(g->Net + 3) / 4, 256, 0, g->stream>>>(G, A);
+  const Bands B = level_bands(g, g->Net);
+  const unsigned nbe = (unsigned)(((int64_t)g->Net * B.nb + 3) / 4);
+  if (B.nb > 1) k_tvd_faces<true><<<nbe, 256, 0, g->stream>>>(G, A, B);
+  else k_tvd_faces<false><<<nbe, 256, 0, g->stream>>>(G, A, B);
   prof_end(g, ps);
   HIPCHK(hipGetLastError());
   return 0;
@@ -161,6 +197,16 @@ static int update_scalars(sunhip_grid *g, const sunhip_scalar_params *sp, const 
     const unsigned nb = (unsigned)((g->Nt + 3) / 4);
     if (srcs)
       k_update_column<NF, 1, true><<<nb, 256, 0, g->stream>>>(g->geo(), A);  // sources: a variant of its own
+    else if (tvd_seg<NF>(g, pre)) {
+      const int ns = (g->maxdepth + SUNHIP_SEG - 1) / SUNHIP_SEG;
+      if (ns <= 8) {
+        if (pre) k_update_column_seg<NF, true, 1><<<g->Nt, ns * 64, 0, g->stream>>>(g->geo(), A);
+        else k_update_column_seg<NF, false, 1><<<g->Nt, ns * 64, 0, g->stream>>>(g->geo(), A);
+      } else if constexpr (NF <= 4) {
+        if (pre) k_update_column_seg<NF, true, 2><<<g->Nt, (ns + 1) / 2 * 64, 0, g->stream>>>(g->geo(), A);
+        else k_update_column_seg<NF, false, 2><<<g->Nt, (ns + 1) / 2 * 64, 0, g->stream>>>(g->geo(), A);
+      }
+    }
     else if (pre && g->tune_tvdgrp == 4) k_update_column<NF, 4, false, true><<<nb, 256, 0, g->stream>>>(g->geo(), A);
     else if (pre && g->tune_tvdgrp == 2 && g->tune_tvdhead == 16)
       k_update_column<NF, 2, false, true, 16><<<nb, 256, 0, g->stream>>>(g->geo(), A);

@@ -45,11 +45,13 @@ struct TvdArgs {
 // pass 1 (main/tvd.c:46-65), cells of celldist[0..2).  The faces' level-
 // invariant data (edge base, df, normal, neighbour base and depth) are read
 // once per column.  NF: faces per cell at most.
+// Levels [ka, kz) only.
 template <int NF, int GRP = 1>
-__device__ __forceinline__ void tvd_sums_tile(const Geo &G, const TvdArgs &A, int t, int l) {
+__device__ __forceinline__ void tvd_sums_tile(const Geo &G, const TvdArgs &A, int t, int l, int ka = 0,
+                                              int kz = 0x7fffffff) {
   if (t >= G.Nt) return;
-  const int s = t * 64 + l, n = G.nk[s];
-  if (n == 0 || G.comp[s] == 0) return;
+  const int s = t * 64 + l, n = min(G.nk[s], kz);
+  if (n <= ka || G.comp[s] == 0) return;
   const int NS = G.NS, nf = G.nf[s];
   const uint32_t base = (uint32_t)(G.toff[t] + l);
   const double th = A.theta;
@@ -72,7 +74,7 @@ __device__ __forceinline__ void tvd_sums_tile(const Geo &G, const TvdArgs &A, in
   // GRP levels at a time: every load of the group first (levels past the
   // column clamped to its last, the neighbour's scalar to its own bottom),
   // then the sums in face order as below
-  const int k1 = G.ctop[s];
+  const int k1 = max(G.ctop[s], ka);
   for (int k0 = k1; k0 < n; k0 += GRP) {
     double vs[GRP], vu[GRP][NF], vt[GRP][NF], vz[GRP][NF], vn[GRP][NF];
 #pragma unroll
@@ -143,25 +145,28 @@ __device__ __forceinline__ void store_terms(const Geo &G, const TvdArgs &A, int 
 // column's flux terms of each level too (store_terms), from the values in
 // registers.  Edges outside the pass (closed boundaries) get theirs from the
 // stored face values, which the column would otherwise read.
-__device__ __forceinline__ void tvd_faces_tile(const Geo &G, const TvdArgs &A, int t, int l) {
+// Levels [ka, kz) only.
+__device__ __forceinline__ void tvd_faces_tile(const Geo &G, const TvdArgs &A, int t, int l, int ka = 0,
+                                               int kz = 0x7fffffff) {
   if (t >= G.Net) return;
   const int s = t * 64 + l, ec = G.e_comp[s];
   const int64_t base = G.eoff[t] + l;
-  const int et = G.e_etop[s], nke = G.e_nke[s];
+  const int nke = min(G.e_nke[s], kz), et = min(G.e_etop[s], kz);
+  if (nke <= ka) return;
   const double th = A.theta;
   const bool terms = A.P1 != nullptr;
   double c1 = 0, c2 = 0;
   if (terms) face_term_consts(G, A, s, c1, c2);
   if (ec == 0) {
     if (terms)
-      for (int k = 0; k < nke; k++) {
+      for (int k = ka; k < nke; k++) {
         const int64_t ei = base + (int64_t)k * 64;
         const double ut2 = A.utmp2[ei];
         store_terms(G, A, s, ei, c1, c2, th * A.u[ei] + (1 - th) * ut2, ut2, A.SfHp[ei], A.SfHm[ei]);
       }
     return;
   }
-  for (int k = 0; k < et; k++) {
+  for (int k = ka; k < et; k++) {
     const int64_t ei = base + (int64_t)k * 64;
     A.SfHp[ei] = A.SfHm[ei] = 0;
     if (terms) {
@@ -171,7 +176,7 @@ __device__ __forceinline__ void tvd_faces_tile(const Geo &G, const TvdArgs &A, i
   }
   if (ec == 1) {
     const int64_t e1 = G.e_c1[s], e2 = G.e_c2[s];
-    for (int k = et; k < nke; k++) {
+    for (int k = max(et, ka); k < nke; k++) {
       const int64_t ei = base + (int64_t)k * 64;
       const double ut2 = A.utmp2[ei];
       const double un = th * A.u[ei] + (1 - th) * ut2;
@@ -189,7 +194,7 @@ __device__ __forceinline__ void tvd_faces_tile(const Geo &G, const TvdArgs &A, i
     }
   } else {
     const int64_t ib = G.e_c1[s];
-    for (int k = et; k < nke; k++) {
+    for (int k = max(et, ka); k < nke; k++) {
       const int64_t ei = base + (int64_t)k * 64;
       const double hp = A.bscal ? A.bscal[ei] : 0.0;
       const double hm = A.s[ib + (int64_t)k * 64];
@@ -720,6 +725,189 @@ __device__ __forceinline__ void update_column_tile(const Geo &G, const ColArgs &
   for (int k = 0; k < ct; k++) A.s[base + (int64_t)k * 64] = 0;
   const double stop = A.s[base + (int64_t)ktop * 64];
   for (int k = ct; k < cto; k++) A.s[base + (int64_t)k * 64] = stop;
+}
+
+// One tile of UpdateScalars without source terms by a block, one wave per
+// SUNHIP_SEG levels (SPW = 1) or two such segments.  Each wave assembles its
+// levels' rows and holds them in registers; the elimination passes from wave
+// to wave through LDS (b, c and d of the row above), the back substitution
+// upward, so no row goes to memory between the sweeps.  Same operations in
+// the same order as update_column_tile: the same bits.  In place is allowed:
+// every wave has read its levels' old values before any result is stored.
+// pass: 4 x 64 values of LDS.  Called by all threads of the block.
+template <int NF, bool PRE, int SPW>
+__device__ __forceinline__ void update_column_seg(const Geo &G, const ColArgs &A, int t, double (*pass)[64]) {
+  constexpr int SG = SUNHIP_SEG * SPW, GR = 2;
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, s = t * 64 + l;
+  const int W = (G.tdep[t] - 1 + SG - 1) / SG;  // waves with levels
+  const int nk = G.nk[s], ct = G.ctop[s], cto = G.ctopold[s], nfs = G.nf[s];
+  const bool own = nk > 0 && G.comp[s] == 1;
+  const int64_t base = nk > 0 ? (int64_t)(G.toff[t] + l) : 0;
+  const int ktop = ct >= cto ? ct : cto, nb = nk - 1 - ktop, k0 = w * SG;
+  const double theta = A.theta, dt = A.dt, td = theta * dt, otd = (1 - theta) * dt;
+  const bool tvdv = A.TVD != 0;
+  const Col dzz{A.dzz, base, nk}, dzo{A.dzzold, base, nk}, so{A.s_old, base, nk};
+  auto kap = [&](int k) { return k < nk ? A.kappa_tv[base + (int64_t)k * 64] : 0.0; };
+  double ra[SG], rb[SG], rc[SG], rd[SG];
+  double cn0 = 0, sold = 0, dznew = 0, dtop = 0;
+#pragma unroll
+  for (int j = 0; j < SG; j++) { ra[j] = 0; rb[j] = 1; rc[j] = 0; rd[j] = 0; }
+  if (own && k0 < nk && k0 + SG > ktop) {
+    FaceC fc[NF];
+    face_consts(G, A, s, G.Ac[s], fc);
+    // the windows at level kf (the first row of this wave), and the face above it
+    const int kf = max(k0, ktop);
+    double s0 = so.at(kf - 1), s1 = so.at(kf), s2 = so.at(kf + 1), s3 = so.at(kf + 2);
+    double z0 = dzz.at(kf), z1 = dzz.at(kf + 1), o0 = dzo.at(kf), o1 = dzo.at(kf + 1);
+    double q0 = kap(kf), q1 = kap(kf + 1);
+    double apN = 0, amN = 0, apO = 0, amO = 0, bd1 = 0;  // at the face below the current level
+    if (kf > ktop) {  // the face above: its windows are one level up
+      const double sm2 = so.at(kf - 2), zu = dzz.at(kf - 1), ou = dzo.at(kf - 1), qu = kap(kf - 1);
+      if (tvdv) {
+        apam(A.wnew[base + (int64_t)kf * 64], z0, zu, sm2, s0, s1, s2, nk, ktop, kf, dt, A.TVD, apN, amN);
+        apam(A.wtmp2[base + (int64_t)kf * 64], o0, ou, sm2, s0, s1, s2, nk, ktop, kf, dt, A.TVD, apO, amO);
+      } else {
+        apam_plain(A.wnew, base, kf, apN, amN);
+        apam_plain(A.wtmp2, base, kf, apO, amO);
+      }
+      bd1 = (2.0 * A.kappa + qu + q0) / (zu + z0);
+    } else {  // the top row folds the levels above it and those the surface crossed
+      dznew = z0;
+      if (ct < cto) {
+        dznew = 0;
+        for (int kk = ct; kk <= cto; kk++) dznew += dzz.at(kk);
+      }
+      dtop = o0 * s1;
+      if (cto <= ct) {
+        dtop = 0;
+        for (int kk = cto; kk <= ct; kk++) dtop += dzo.at(kk) * so.at(kk);
+      }
+      for (int kk = 0; kk <= ktop && kk < nk; kk++) cn0 -= hflux<NF, PRE>(A, fc, nfs, kk);
+      sold = s1;
+    }
+#pragma unroll
+    for (int g = 0; g < SG; g += GR) {
+      LevelIn<NF> L[GR];
+#pragma unroll
+      for (int j = 0; j < GR; j++) {
+        const int k = k0 + g + j;
+        load_level<NF, false, PRE>(A, fc, base, nk, k < ktop ? ktop : (k < nk ? k : nk - 1), L[j]);
+      }
+#pragma unroll
+      for (int j = 0; j < GR; j++) {
+        const int k = k0 + g + j;
+        if (k < ktop || k >= nk) continue;
+        const double apN_k = apN, amN_k = amN, apO_k = apO, amO_k = amO, bd_k = bd1;
+        if (tvdv) {
+          apam(L[j].wn, z1, z0, s0, s1, s2, s3, nk, ktop, k + 1, dt, A.TVD, apN, amN);
+          apam(L[j].wo, o1, o0, s0, s1, s2, s3, nk, ktop, k + 1, dt, A.TVD, apO, amO);
+        } else {
+          apN = 0.5 * (L[j].wn + fabs(L[j].wn));
+          amN = 0.5 * (L[j].wn - fabs(L[j].wn));
+          apO = 0.5 * (L[j].wo + fabs(L[j].wo));
+          amO = 0.5 * (L[j].wo - fabs(L[j].wo));
+        }
+        bd1 = (k + 1 < nk) ? (2.0 * A.kappa + q0 + q1) / (z0 + z1) : 0.0;
+        const double sk = s1, skm = s0, skp = s2;
+        double a, b, c, d;
+        if (k == ktop) {
+          a = 0;
+          b = dznew - td * amN;
+          c = -td * apN;
+          if (nb == 0) b += c;
+          if (ktop < nk - 1) {
+            b += td * (bd1 + 2 * A.alpha_top * bd1);
+            c -= td * bd1;
+          }
+          d = dtop;
+          if (ktop < nk - 1)
+            d = d - otd * (-amO * sk - apO * skp) + otd * (-(2 * A.alpha_top * bd1 + bd1) * sk + bd1 * skp);
+          d += cn0;
+        } else {
+          a = td * amN_k;
+          b = z0 + td * (apN_k - amN);
+          c = -td * apN;
+          d = o0 * sk;
+          if (k == nk - 1) {
+            b += c;
+            a -= td * bd_k;
+            b += td * (bd_k + 2 * A.alpha_bot * bd_k);
+            d -= otd * (amO_k * skm + apO_k * sk) - otd * (bd_k * skm - (bd_k + 2 * A.alpha_bot * bd_k) * sk);
+          } else {
+            a -= td * bd_k;
+            b += td * (bd_k + bd1);
+            c -= td * bd1;
+            d -= otd * (amO_k * skm + (apO_k - amO) * sk - apO * skp) -
+                 otd * (bd_k * skm - (bd_k + bd1) * sk + bd1 * skp);
+          }
+          const double cnk = -hflux_in<NF, PRE>(A, fc, nfs, k, L[j]);
+          d += cnk;
+          A.Cn[base + (int64_t)k * 64] = cnk;
+        }
+        ra[g + j] = a; rb[g + j] = b; rc[g + j] = c; rd[g + j] = d;
+        s0 = s1; s1 = s2; s2 = s3; s3 = L[j].sn;
+        z0 = z1; z1 = L[j].zn;
+        o0 = o1; o1 = L[j].on;
+        q0 = q1; q1 = L[j].qn;
+      }
+    }
+  }
+  // elimination, top down; rows outside [ktop, nk) are a = c = d = 0, b = 1 and
+  // change nothing
+  for (int v = 0; v < W; v++) {
+    if (w == v) {
+      double bp = 1, cp = 0, dp = 0;
+      if (v) { bp = pass[0][l]; cp = pass[1][l]; dp = pass[2][l]; }
+#pragma unroll
+      for (int j = 0; j < SG; j++) {
+        const int k = k0 + j;
+        if (k > ktop && k < nk) {
+          rb[j] -= ra[j] * cp / bp;
+          rd[j] -= ra[j] * dp / bp;
+        }
+        bp = rb[j]; cp = rc[j]; dp = rd[j];
+      }
+      pass[0][l] = bp; pass[1][l] = cp; pass[2][l] = dp;
+    }
+    __syncthreads();
+  }
+  // d/b of every row ahead of the upward chain
+#pragma unroll
+  for (int j = 0; j < SG; j++) ra[j] = rd[j] / rb[j];
+  for (int v = W - 1; v >= 0; v--) {
+    if (w == v) {
+      double un = v < W - 1 ? pass[0][l] : 0.0;
+#pragma unroll
+      for (int j = SG - 1; j >= 0; j--) {
+        const int k = k0 + j;
+        if (own && k >= ktop && k < nk) {
+          un = k == nk - 1 ? ra[j] : ra[j] - rc[j] * un / rb[j];
+          rd[j] = un;
+          if (k == ktop) {  // to the levels above it
+            if (nb == 0) un = A.step > 1 ? ((rb[j] > 0 && A.active[s] != 0) ? ra[j] : 0) : sold;
+            rd[j] = un;
+            pass[1][l] = cn0;
+            pass[3][l] = un;
+          }
+        }
+      }
+      pass[0][l] = un;
+    }
+    __syncthreads();
+  }
+  if (!own || k0 >= nk) return;
+  const double stop = pass[3][l], ctopv = pass[1][l] / (1 + abs(ct - ktop));
+#pragma unroll
+  for (int j = 0; j < SG; j++) {
+    const int k = k0 + j;
+    const int64_t idx = base + (int64_t)k * 64;
+    if (k >= nk) continue;
+    // above ktop the surface's value down to ctop, 0 over it; Cn folds its
+    // top value over [ctop, ktop]
+    const double sv = k < ct ? 0.0 : (k < cto ? stop : rd[j]);
+    if (k != ktop || nb > 0 || A.step > 1 || k < cto) A.s[idx] = sv;
+    if (k <= ktop) A.Cn[idx] = k < ct ? 0.0 : ctopv;
+  }
 }
 
 // Both passes of HorizontalFaceScalars (sums, then limited face values) for
