@@ -120,7 +120,8 @@ struct sunhip_grid {
   int Nt = 0, Net = 0, NS = 0, NES = 0;
   int64_t NT = 0, NE = 0;           // padded element counts (cells, edges)
   int64_t Nflat = 0, NflatW = 0, NflatE = 0;
-  int maxdepth = 0;                 // deepest tile
+  int maxdepth = 0;                 // deepest column
+  int maxedepth = 0;                // most levels an edge tile stores
   std::vector<int> slot_of_cell, cell_of_slot, slot_of_edge, edge_of_slot;
   std::vector<int> toff, tdep, eoff, edep;
   std::vector<int> Nk, Nkc;         // host copies
