@@ -14,13 +14,30 @@
 
 using namespace sunhip;
 
-template <int NF>
-__global__ __launch_bounds__(256) void k_qsource(Geo G, StepArgs A) {
-  qsource_tile<NF>(G, A, xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), threadIdx.x & 63);
+// BAND: a wave per tile and band of levels (Bands), else one per tile.  The
+// lock exchange (32 tiles of 50 levels): source 51 -> 10 us, Corrector 54 -> 9,
+// Continuity 70 -> 17.
+template <int NF, bool BAND>
+__global__ __launch_bounds__(256) void k_qsource(Geo G, StepArgs A, Bands B) {
+  const int v = xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
+  if (!BAND) { qsource_tile<NF>(G, A, v, l); return; }
+  const int t = v / B.nb, k0 = (v - t * B.nb) * B.len;
+  qsource_tile<NF>(G, A, t, l, k0, k0 + B.len);
 }
 
-__global__ __launch_bounds__(256) void k_corrector(Geo G, StepArgs A) {
-  corrector_tile(G, A, xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), threadIdx.x & 63);
+template <bool BAND>
+__global__ __launch_bounds__(256) void k_corrector(Geo G, StepArgs A, Bands B) {
+  const int v = xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
+  if (!BAND) { corrector_tile(G, A, v, l); return; }
+  const int t = v / B.nb, k0 = (v - t * B.nb) * B.len;
+  corrector_tile(G, A, t, l, k0, k0 + B.len);
+}
+
+// one block per tile, one wave per SUNHIP_SEG levels
+template <int NF>
+__global__ __launch_bounds__(1024) void k_continuity_seg(Geo G, StepArgs A) {
+  __shared__ double carry[64];
+  continuity_seg<NF>(G, A, xcd_block(blockIdx.x, gridDim.x), carry);
 }
 
 template <int NF>
@@ -64,10 +81,13 @@ int sunhip_compute_qsource(sunhip_grid *g, double theta, double dt, const char *
   int rc = step_args(g, theta, dt, "q", "qp", "w", src, &A);
   if (rc) return rc;
   const Geo G = g->geo();
-  const int nb = (std::max(g->Nt, g->Net) + 3) / 4;
+  const int tiles = std::max(g->Nt, g->Net), nb = (tiles + 3) / 4;
+  const Bands B = level_bands(g, tiles);
   const int ps = prof_begin(g, PK_QSOURCE);
   with_nf(g->mf, [&](auto nf) {
-    k_qsource<decltype(nf)::value><<<nb, 256, 0, g->stream>>>(G, A);
+    constexpr int NF = decltype(nf)::value;
+    if (B.nb > 1) k_qsource<NF, true><<<(tiles * B.nb + 3) / 4, 256, 0, g->stream>>>(g->geo(), A, B);
+    else k_qsource<NF, false><<<nb, 256, 0, g->stream>>>(g->geo(), A, B);
     return 0;
   });
   prof_end(g, ps);
@@ -80,9 +100,11 @@ int sunhip_corrector(sunhip_grid *g, double dt, const char *qc, const char *q) {
   StepArgs A;
   int rc = step_args(g, 1.0, dt, qc, q, "w", "src", &A);
   if (rc) return rc;
-  const int nb = (std::max(g->Nt, g->Net) + 3) / 4;
+  const int tiles = std::max(g->Nt, g->Net);
+  const Bands B = level_bands(g, tiles);
   const int ps = prof_begin(g, PK_CORRECT);
-  k_corrector<<<nb, 256, 0, g->stream>>>(g->geo(), A);
+  if (B.nb > 1) k_corrector<true><<<(tiles * B.nb + 3) / 4, 256, 0, g->stream>>>(g->geo(), A, B);
+  else k_corrector<false><<<(tiles + 3) / 4, 256, 0, g->stream>>>(g->geo(), A, B);
   prof_end(g, ps);
   HIPCHK(hipGetLastError());
   return 0;
@@ -96,8 +118,15 @@ int sunhip_continuity(sunhip_grid *g, double theta, const char *w) {
   const Geo G = g->geo();
   const int nb = (g->Nt + 3) / 4;
   const int ps = prof_begin(g, PK_CONTINUITY);
+  const int ns = (g->maxdepth + SUNHIP_SEG - 1) / SUNHIP_SEG;
   with_nf(g->mf, [&](auto nf) {
-    k_continuity<decltype(nf)::value><<<nb, 256, 0, g->stream>>>(G, A);
+    constexpr int NF = decltype(nf)::value;
+    if constexpr (NF <= 4)
+      if (g->Nt <= 1024 && ns <= 16) {
+        k_continuity_seg<NF><<<g->Nt, ns * 64, 0, g->stream>>>(G, A);
+        return 0;
+      }
+    k_continuity<NF><<<nb, 256, 0, g->stream>>>(G, A);
     return 0;
   });
   prof_end(g, ps);

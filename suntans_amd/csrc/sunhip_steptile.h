@@ -51,17 +51,20 @@ struct ColFaces {
 };
 
 // ComputeQSource: src over [ctop, Nk) of every column (zero outside the
-// computational cells); D = df/dg on every edge.
+// computational cells); D = df/dg on every edge.  Levels [ka, kz) only (D with
+// the first).
 template <int NF>
-__device__ __forceinline__ void qsource_tile(const Geo &G, const StepArgs &A, int t, int l) {
-  if (t < G.Net) {
+__device__ __forceinline__ void qsource_tile(const Geo &G, const StepArgs &A, int t, int l, int ka = 0,
+                                             int kz = 0x7fffffff) {
+  if (t < G.Net && ka == 0) {
     const int s = t * 64 + l;
     if (G.e_nkc[s] > 0) A.D[s] = G.df[s] / G.dg[s];
   }
   if (t >= G.Nt) return;
-  const int s = t * 64 + l, n = G.nk[s];
-  if (n == 0) return;
-  const int kt = G.ctop[s];
+  const int s = t * 64 + l, n = min(G.nk[s], kz);
+  if (n <= ka) return;
+  const int kt = max(G.ctop[s], ka);
+  if (kt >= n) return;
   const uint32_t base = (uint32_t)(G.toff[t] + l);
   if (G.comp[s] != 1) {
     for (int k = kt; k < n; k++) at32(A.src, base + (uint32_t)k * 64u) = 0;
@@ -110,16 +113,17 @@ __device__ __forceinline__ void qsource_tile(const Geo &G, const StepArgs &A, in
 
 // Corrector: u on computational interior edges with D != 0 and more than one
 // layer; w of computational columns (surface ghost -qc[ctop]); q += qc on
-// columns of more than one layer.
-__device__ __forceinline__ void corrector_tile(const Geo &G, const StepArgs &A, int t, int l) {
+// columns of more than one layer.  Levels [ka, kz) only.
+__device__ __forceinline__ void corrector_tile(const Geo &G, const StepArgs &A, int t, int l, int ka = 0,
+                                               int kz = 0x7fffffff) {
   const double dt = A.dt;
   if (t < G.Net) {
     const int s = t * 64 + l;
     const int et = G.e_etop[s], nke = G.e_nke[s];
-    if (G.e_comp[s] == 1 && A.D[s] != 0 && et < nke - 1) {
+    if (G.e_comp[s] == 1 && A.D[s] != 0 && et < nke - 1 && max(et, ka) < min(nke, kz)) {
       const uint32_t base = (uint32_t)(G.eoff[t] + l), c1 = (uint32_t)G.e_c1[s], c2 = (uint32_t)G.e_c2[s];
       const double f = dt / G.dg[s];
-      for (int k = et; k < nke; k++) {
+      for (int k = max(et, ka); k < min(nke, kz); k++) {
         const uint32_t k64 = (uint32_t)k * 64u;
         at32(A.u, base + k64) -= f * (at32(A.qc, c1 + k64) - at32(A.qc, c2 + k64));
       }
@@ -128,20 +132,21 @@ __device__ __forceinline__ void corrector_tile(const Geo &G, const StepArgs &A, 
   if (t >= G.Nt) return;
   const int s = t * 64 + l, n = G.nk[s];
   if (n == 0 || G.comp[s] != 1) return;
-  const int kt = G.ctop[s];
-  const uint32_t base = (uint32_t)(G.toff[t] + l);
-  double qprev = at32(A.qc, base + (uint32_t)kt * 64u), dprev = at32(A.dzz, base + (uint32_t)kt * 64u);
-  const double qtop = qprev, dtop = dprev;
-  for (int k = kt + 1; k < n; k++) {
+  const int kt = G.ctop[s], ks = max(kt + 1, ka), ke = min(n, kz);
+  if (ke <= ka || ke <= kt) return;
+  const uint32_t base = (uint32_t)(G.toff[t] + l), ip = base + (uint32_t)(ks - 1) * 64u;
+  double qprev = at32(A.qc, ip), dprev = at32(A.dzz, ip);
+  const double qtop = qprev, dtop = dprev;  // of level kt in its own band
+  for (int k = ks; k < ke; k++) {
     const uint32_t idx = base + (uint32_t)k * 64u;
     const double qk = at32(A.qc, idx), dk = at32(A.dzz, idx);
     at32(A.w, idx) -= 2.0 * dt / (dprev + dk) * (qprev - qk);
     qprev = qk;
     dprev = dk;
   }
-  at32(A.w, base + (uint32_t)kt * 64u) += 2.0 * dt / dtop * qtop;
+  if (kt >= ka) at32(A.w, base + (uint32_t)kt * 64u) += 2.0 * dt / dtop * qtop;
   if (kt < n - 1)
-    for (int k = kt; k < n; k++) {
+    for (int k = max(kt, ka); k < ke; k++) {
       const uint32_t idx = base + (uint32_t)k * 64u;
       at32(A.q, idx) += at32(A.qc, idx);
     }
@@ -195,6 +200,65 @@ __device__ __forceinline__ void continuity_tile(const Geo &G, const StepArgs &A,
       wk1 = v;
       w2k1 = w2[j];
     }
+  }
+}
+
+// Continuity of one tile by a block, one wave per SUNHIP_SEG levels: each wave
+// forms its levels' face terms, then the upward sum passes from wave to wave
+// (carry, 64 values of LDS).  Same operations in the same order as
+// continuity_tile.
+template <int NF>
+__device__ __forceinline__ void continuity_seg(const Geo &G, const StepArgs &A, int t, double *carry) {
+  constexpr int SG = SUNHIP_SEG;
+  const int wv = threadIdx.x >> 6, l = threadIdx.x & 63, s = t * 64 + l, k0 = wv * SG;
+  const int W = (G.tdep[t] - 1 + SG - 1) / SG;  // waves with levels
+  const int n = G.nk[s], kt = G.ctop[s], nf = G.nf[s];
+  const bool own = n > 0 && G.comp[s] == 1;
+  const uint32_t base = n > 0 ? (uint32_t)(G.toff[t] + l) : 0u;
+  const double th = A.theta, tf = (1 - th) / th;
+  double w2[SG + 1], tm[SG][NF];
+  int nke[NF];
+  if (own && k0 < n) {
+    ColFaces<NF> F;
+    F.load(G, s, nf);
+    const double Ac = G.Ac[s];
+#pragma unroll
+    for (int f = 0; f < NF; f++) nke[f] = f < nf ? F.nke[f] : 0;
+#pragma unroll
+    for (int j = 0; j <= SG; j++) w2[j] = at32(A.wtmp2, base + (uint32_t)min(k0 + j, n) * 64u);
+#pragma unroll
+    for (int j = 0; j < SG; j++)
+#pragma unroll
+      for (int f = 0; f < NF; f++) {
+        tm[j][f] = 0;
+        if (k0 + j < nke[f]) {
+          const uint32_t ei = F.eb[f] + (uint32_t)(k0 + j) * 64u;
+          tm[j][f] = (th * at32(A.u, ei) + (1 - th) * at32(A.utmp2, ei)) * F.df[f] * F.nrm[f] / Ac / th *
+                     at32(A.dzf, ei);
+        }
+      }
+  }
+  for (int v = W - 1; v >= 0; v--) {
+    if (wv == v && own && k0 < n) {
+      double wk1 = k0 + SG < n ? carry[l] : 0.0;
+      if (k0 + SG >= n) at32(A.w, base + (uint32_t)n * 64u) = 0;
+#pragma unroll
+      for (int j = SG - 1; j >= 0; j--) {
+        const int k = k0 + j;
+        if (k >= n) continue;
+        double x = 0;
+        if (k >= kt) {
+          x = wk1 - tf * (w2[j] - w2[j + 1]);
+#pragma unroll
+          for (int f = 0; f < NF; f++)
+            if (k < nke[f]) x -= tm[j][f];
+          wk1 = x;
+        }
+        at32(A.w, base + (uint32_t)k * 64u) = x;
+      }
+      carry[l] = wk1;
+    }
+    __syncthreads();
   }
 }
 

@@ -16,14 +16,17 @@
 
 using namespace sunhip;
 
-__global__ __launch_bounds__(256) void k_upred_cells(Geo G, UPArgs A) {
-  upred_cells_tile(G, A, xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), threadIdx.x & 63);
+// The level-wise kernels run one wave per tile and band of levels (Bands).
+__global__ __launch_bounds__(256) void k_upred_cells(Geo G, UPArgs A, Bands B) {
+  const int v = xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), t = v / B.nb, k0 = (v - t * B.nb) * B.len;
+  upred_cells_tile(G, A, t, threadIdx.x & 63, k0, k0 + B.len);
 }
 __global__ __launch_bounds__(256) void k_upred_edges(Geo G, UPArgs A) {
   upred_edge_tile(G, A, xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), threadIdx.x & 63);
 }
-__global__ __launch_bounds__(256) void k_upred_hterm(Geo G, UPArgs A) {
-  upred_hterm_tile(G, A, xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), threadIdx.x & 63);
+__global__ __launch_bounds__(256) void k_upred_hterm(Geo G, UPArgs A, Bands B) {
+  const int v = xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), t = v / B.nb, k0 = (v - t * B.nb) * B.len;
+  upred_hterm_tile(G, A, t, threadIdx.x & 63, k0, k0 + B.len);
 }
 template <int NF>
 __global__ __launch_bounds__(256) void k_upred_htmp(Geo G, UPArgs A) {
@@ -32,8 +35,9 @@ __global__ __launch_bounds__(256) void k_upred_htmp(Geo G, UPArgs A) {
 __global__ __launch_bounds__(256) void k_upred_dry(Geo G, UPArgs A) {
   upred_dry_tile(G, A, xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), threadIdx.x & 63);
 }
-__global__ __launch_bounds__(256) void k_upred_velocity(Geo G, UPArgs A) {
-  upred_velocity_tile(G, A, xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), threadIdx.x & 63);
+__global__ __launch_bounds__(256) void k_upred_velocity(Geo G, UPArgs A, Bands B) {
+  const int v = xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), t = v / B.nb, k0 = (v - t * B.nb) * B.len;
+  upred_velocity_tile(G, A, t, threadIdx.x & 63, k0, k0 + B.len);
 }
 
 namespace sunhip {
@@ -76,7 +80,8 @@ int sunhip_u_predict(sunhip_grid *g, const sunhip_upred_params *p) {
   if (rc) return rc;
   HIPCHK(hipMemsetAsync(A.err, 0, 2 * sizeof(int), g->stream));
   const Geo G = g->geo();
-  k_upred_cells<<<(g->Nt + 3) / 4, 256, 0, g->stream>>>(G, A);
+  const Bands B = level_bands(g, g->Nt);
+  k_upred_cells<<<(g->Nt * B.nb + 3) / 4, 256, 0, g->stream>>>(G, A, B);
   k_upred_edges<<<(g->Net + 3) / 4, 256, 0, g->stream>>>(G, A);
   HIPCHK(hipGetLastError());
   int err[2] = {0, 0};
@@ -93,7 +98,8 @@ int sunhip_u_solve(sunhip_grid *g, const sunhip_upred_params *p, const sunhip_cg
   int rc = upred_args(g, p, &A);
   if (rc) return rc;
   const Geo G = g->geo();
-  k_upred_hterm<<<(g->Net + 3) / 4, 256, 0, g->stream>>>(G, A);
+  const Bands B = level_bands(g, g->Net);
+  k_upred_hterm<<<(g->Net * B.nb + 3) / 4, 256, 0, g->stream>>>(G, A, B);
   with_nf(g->mf, [&](auto nf) {
     k_upred_htmp<decltype(nf)::value><<<(g->Nt + 3) / 4, 256, 0, g->stream>>>(G, A);
     return 0;
@@ -101,7 +107,7 @@ int sunhip_u_solve(sunhip_grid *g, const sunhip_upred_params *p, const sunhip_cg
   HIPCHK(hipGetLastError());
   if ((rc = sunhip_h_solve(g, prm, p->grav, p->theta, p->dt, st))) return rc;
   k_upred_dry<<<(g->Nt + 3) / 4, 256, 0, g->stream>>>(G, A);
-  k_upred_velocity<<<(g->Net + 3) / 4, 256, 0, g->stream>>>(G, A);
+  k_upred_velocity<<<(g->Net * B.nb + 3) / 4, 256, 0, g->stream>>>(G, A, B);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(g->stream));
   return 0;

@@ -36,13 +36,13 @@ struct UPArgs {
   int *err;  // [0]: a level of an edge with two zero-height cells; [1]: U*** = nan
 };
 
-// wtmp2 = w on every column (main/phys.c:2597-2599).
-__device__ __forceinline__ void upred_cells_tile(const Geo &G, const UPArgs &A, int t, int l) {
+// wtmp2 = w on every column (main/phys.c:2597-2599), levels [ka, kz).
+__device__ __forceinline__ void upred_cells_tile(const Geo &G, const UPArgs &A, int t, int l, int ka, int kz) {
   if (t >= G.Nt) return;
   const int s = t * 64 + l, n = G.nk[s];
   if (n == 0) return;
   const uint32_t base = (uint32_t)(G.toff[t] + l);
-  for (int k = 0; k <= n; k++) at32(A.wtmp2, base + (uint32_t)k * 64u) = at32(A.w, base + (uint32_t)k * 64u);
+  for (int k = ka; k <= min(n, kz - 1); k++) at32(A.wtmp2, base + (uint32_t)k * 64u) = at32(A.w, base + (uint32_t)k * 64u);
 }
 
 // Everything of UPredictor before the open-boundary hooks for edge slot
@@ -251,14 +251,14 @@ __device__ __forceinline__ void upred_edge_tile(const Geo &G, const UPArgs &A, i
 // as +1: with -1 it is the same value negated, exactly, so a cell adds
 // normal * hterm.  One lane per edge walks its levels (coalesced), and the
 // cell sum reads one value per face and level instead of gathering u, utmp
-// and dzf.
-__device__ __forceinline__ void upred_hterm_tile(const Geo &G, const UPArgs &A, int t, int l) {
+// and dzf.  Levels [ka, kz).
+__device__ __forceinline__ void upred_hterm_tile(const Geo &G, const UPArgs &A, int t, int l, int ka, int kz) {
   if (t >= G.Net) return;
-  const int s = t * 64 + l, ne = G.e_nke[s];
-  if (ne == 0) return;
+  const int s = t * 64 + l, ne = min(G.e_nke[s], kz);
+  if (ne <= ka) return;
   const uint32_t base = (uint32_t)(G.eoff[t] + l);
   const double th = A.theta, df = G.df[s];
-  for (int k = G.e_etop[s]; k < ne; k++) {
+  for (int k = max(G.e_etop[s], ka); k < ne; k++) {
     const uint32_t ei = base + (uint32_t)k * 64u;
     at32(A.hterm, ei) = ((1 - th) * at32(A.u, ei) + th * at32(A.utmp, ei)) * df * at32(A.dzf, ei);
   }
@@ -279,7 +279,16 @@ __device__ __forceinline__ void upred_htmp_tile(const Geo &G, const UPArgs &A, i
       const int es = G.es[f * NS + s];
       const uint32_t eb = (uint32_t)G.eb[f * NS + s];
       const double nrm = (double)G.nrm[f * NS + s];
-      for (int k = G.e_etop[es]; k < G.e_nke[es]; k++) sum += nrm * at32(A.hterm, eb + (uint32_t)k * 64u);
+      // eight values loaded, then added in turn
+      const int e0 = G.e_etop[es], e1 = G.e_nke[es];
+      for (int kb = e0; kb < e1; kb += 8) {
+        double v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = at32(A.hterm, eb + (uint32_t)min(kb + j, e1 - 1) * 64u);
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+          if (kb + j < e1) sum += nrm * v[j];
+      }
     }
   }
   A.htmp[s] = G.Ac[s] * A.h[s] - A.dt * sum;
@@ -301,19 +310,19 @@ __device__ __forceinline__ void upred_dry_tile(const Geo &G, const UPArgs &A, in
 }
 
 // u = U*** - g theta dt E (h1 - h2)/dg on computational edges, zero on a
-// dry one-layer edge (main/phys.c:3008-3018).
-__device__ __forceinline__ void upred_velocity_tile(const Geo &G, const UPArgs &A, int t, int l) {
+// dry one-layer edge (main/phys.c:3008-3018).  Levels [ka, kz).
+__device__ __forceinline__ void upred_velocity_tile(const Geo &G, const UPArgs &A, int t, int l, int ka, int kz) {
   if (t >= G.Net) return;
   const int s = t * 64 + l;
   if (G.e_comp[s] != 1) return;
   const uint32_t base = (uint32_t)(G.eoff[t] + l);
   const int et = G.e_etop[s], ne = G.e_nke[s], s1 = G.e_s1[s], s2 = G.e_s2[s];
   const double hd = A.h[s1] - A.h[s2], dg = G.dg[s];
-  for (int k = et; k < ne; k++) {
+  for (int k = max(et, ka); k < min(ne, kz); k++) {
     const uint32_t ei = base + (uint32_t)k * 64u;
     at32(A.u, ei) = at32(A.utmp, ei) - A.grav * A.theta * A.dt * at32(A.E, ei) * hd / dg;
   }
-  if (et == ne - 1 && at32(A.dzz, (uint32_t)G.e_c1[s] + (uint32_t)et * 64u) == 0 &&
+  if (et >= ka && et < kz && et == ne - 1 && at32(A.dzz, (uint32_t)G.e_c1[s] + (uint32_t)et * 64u) == 0 &&
       at32(A.dzz, (uint32_t)G.e_c2[s] + (uint32_t)et * 64u) == 0)
     at32(A.u, base + (uint32_t)et * 64u) = 0;
 }

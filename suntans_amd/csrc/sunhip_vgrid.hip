@@ -134,28 +134,36 @@ __global__ __launch_bounds__(256) void k_sfh_bottom(Geo G, VGArgs A) {
 }
 
 // SetFluxHeight, one lane per edge (main/phys.c:4342-4344, 4351-4427).
-__global__ __launch_bounds__(256) void k_sfh_edges(Geo G, VGArgs A) {
-  const int t = xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
+// Each level's value is formed at once (the reference clears, fills, sets the
+// bottom one and clears the small ones in turn), in bands of levels.
+__global__ __launch_bounds__(256) void k_sfh_edges(Geo G, VGArgs A, Bands B) {
+  const int v = xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
+  const int t = v / B.nb, ka = (v - t * B.nb) * B.len, kz = ka + B.len;
   if (t >= G.Net) return;
   const int s = t * 64 + l, nkc = G.e_nkc[s];
   if (nkc == 0) return;
   const uint32_t base = (uint32_t)(G.eoff[t] + l);
-  auto F = [&](int k) -> double & { return at32(A.dzf, base + (uint32_t)k * 64u); };
-  for (int k = 0; k < nkc; k++) F(k) = 0;
   int s1 = G.e_s1[s], s2 = G.e_s2[s], b1 = G.e_c1[s], b2 = G.e_c2[s];
   if (s1 < 0) { s1 = s2; b1 = b2; }
   if (s2 < 0) { s2 = s1; b2 = b1; }
   const int et = A.etop[s], ne = G.e_nke[s];
   auto Z1 = [&](int k) { return at32(A.dzz, (uint32_t)b1 + (uint32_t)k * 64u); };
   auto Z2 = [&](int k) { return at32(A.dzz, (uint32_t)b2 + (uint32_t)k * 64u); };
-  for (int k = et; k < ne; k++) F(k) = vupwind(at32(A.u, base + (uint32_t)k * 64u), Z1(k), Z2(k));
-  const int k = ne - 1;
-  if (et == k)
-    F(k) = vmax(0, vupwind(at32(A.u, base + (uint32_t)k * 64u), A.h[s1], A.h[s2]) + vmin(A.dv[s1], A.dv[s2]));
-  else
-    F(k) = vmin(Z1(k), Z2(k));
-  for (int kk = et; kk < ne; kk++)
-    if (F(kk) <= 1e-10) F(kk) = 0;
+  for (int k = ka; k < min(nkc, kz); k++) {
+    const uint32_t idx = base + (uint32_t)k * 64u;
+    double f = 0;
+    if (k >= et && k < ne) {
+      f = vupwind(at32(A.u, idx), Z1(k), Z2(k));
+      if (k == ne - 1) {
+        if (et == k) f = vmax(0, vupwind(at32(A.u, idx), A.h[s1], A.h[s2]) + vmin(A.dv[s1], A.dv[s2]));
+        else f = vmin(Z1(k), Z2(k));
+      }
+      if (f <= 1e-10) f = 0;
+    } else if (k == ne - 1) {
+      f = vmin(Z1(k), Z2(k));  // etop below the bottom face
+    }
+    at32(A.dzf, idx) = f;
+  }
 }
 
 namespace sunhip {
@@ -210,9 +218,10 @@ int sunhip_set_flux_height(sunhip_grid *g, const sunhip_vgrid_params *vp) {
   int rc = vg_args(g, vp, &A);
   if (rc) return rc;
   const Geo G = g->geo();
-  const int nc = (g->Nt + 3) / 4, ne = (g->Net + 3) / 4;
+  const int nc = (g->Nt + 3) / 4;
   if (vp->smoothbot) k_sfh_bottom<true><<<nc, 256, 0, g->stream>>>(G, A);
-  k_sfh_edges<<<ne, 256, 0, g->stream>>>(G, A);
+  const Bands B = level_bands(g, g->Net);
+  k_sfh_edges<<<(g->Net * B.nb + 3) / 4, 256, 0, g->stream>>>(G, A, B);
   if (vp->smoothbot) k_sfh_bottom<false><<<nc, 256, 0, g->stream>>>(G, A);
   HIPCHK(hipGetLastError());
   return 0;

@@ -53,14 +53,17 @@ __device__ __forceinline__ double wupwind(double u, double a, double b) {       
 }  // namespace sunhip
 
 // wc on every column from its top cell down (main/phys.c:2096-2100).
-__global__ __launch_bounds__(256) void k_wp_centres(Geo G, WPArgs A) {
-  const int t = xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
+template <bool BAND>
+__global__ __launch_bounds__(256) void k_wp_centres(Geo G, WPArgs A, Bands B) {
+  const int v = xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
+  const int t = BAND ? v / B.nb : v, ka = BAND ? (v - t * B.nb) * B.len : 0, kz = BAND ? ka + B.len : 0x7fffffff;
   if (t >= G.Nt) return;
   const int s = t * 64 + l, n = G.nk[s];
-  if (n == 0) return;
+  const int kb = max(G.ctop[s], ka), ke = min(n, kz);
+  if (n == 0 || kb >= ke) return;
   const uint32_t base = (uint32_t)(G.toff[t] + l);
-  double wk = at32(A.w, base + (uint32_t)G.ctop[s] * 64u);
-  for (int k = G.ctop[s]; k < n; k++) {
+  double wk = at32(A.w, base + (uint32_t)kb * 64u);
+  for (int k = kb; k < ke; k++) {
     const double wn = at32(A.w, base + (uint32_t)(k + 1) * 64u);
     at32(A.wc, base + (uint32_t)k * 64u) = 0.5 * (wk + wn);
     wk = wn;
@@ -72,13 +75,15 @@ __global__ __launch_bounds__(256) void k_wp_centres(Geo G, WPArgs A) {
 // reference's last loop overwrites them); computational edges take the
 // scheme's value below the deeper top; type-2 edges the boundary row on
 // inflow.  Type-4 edges are refused by the host.  Other edges keep theirs.
-__global__ __launch_bounds__(256) void k_wp_faces(Geo G, WPArgs A) {
-  const int t = xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
+template <bool BAND>
+__global__ __launch_bounds__(256) void k_wp_faces(Geo G, WPArgs A, Bands B) {
+  const int v = xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
+  const int t = BAND ? v / B.nb : v, ka = BAND ? (v - t * B.nb) * B.len : 0, kz = BAND ? ka + B.len : 0x7fffffff;
   if (t >= G.Net) return;
   const int s = t * 64 + l;
   if (G.e_nkc[s] == 0) return;  // padding
   const uint32_t base = (uint32_t)(G.eoff[t] + l);
-  const int s1 = G.e_s1[s], s2 = G.e_s2[s], nke = G.e_nke[s], comp = G.e_comp[s];
+  const int s1 = G.e_s1[s], s2 = G.e_s2[s], nke = min(G.e_nke[s], kz), comp = G.e_comp[s];
   const uint32_t c1 = (uint32_t)G.e_c1[s], c2 = (uint32_t)G.e_c2[s];
   auto E = [&](const double *p, int k) { return at32(p, base + (uint32_t)k * 64u); };
   auto F = [&](int k) -> double & { return at32(A.uf, base + (uint32_t)k * 64u); };
@@ -87,11 +92,11 @@ __global__ __launch_bounds__(256) void k_wp_faces(Geo G, WPArgs A) {
   const bool type3 = s1 >= 0 && s2 >= 0 && (G.comp[s1] == 2 || G.comp[s2] == 2);
   if (type3 || comp == 1) {
     const int kmin = G.ctop[s1] > G.ctop[s2] ? G.ctop[s1] : G.ctop[s2];
-    for (int k = 0; k < kmin; k++) F(k) = 0;
+    for (int k = ka; k < min(kmin, kz); k++) F(k) = 0;
     const int scheme = type3 ? 1 : A.scheme;
     double d1 = 0, d2 = 0;
     if (scheme == 2) { d1 = A.def1[s]; d2 = G.dg[s] - d1; }
-    for (int k = kmin; k < nke; k++) {
+    for (int k = max(kmin, ka); k < nke; k++) {
       const double U = E(A.U, k);
       double v;
       if (scheme == 2) {
@@ -106,7 +111,7 @@ __global__ __launch_bounds__(256) void k_wp_faces(Geo G, WPArgs A) {
       F(k) = v;
     }
   } else if (comp == 2) {
-    for (int k = G.e_etop[s]; k < nke; k++) F(k) = E(A.U, k) > 0 ? E(A.bw, k) : W1(k);
+    for (int k = max(G.e_etop[s], ka); k < nke; k++) F(k) = E(A.U, k) > 0 ? E(A.bw, k) : W1(k);
   }
 }
 
@@ -114,12 +119,14 @@ __global__ __launch_bounds__(256) void k_wp_faces(Geo G, WPArgs A) {
 // on computational columns the horizontal advection through every face
 // (face order) and the vertical advection of w^2, then the horizontal
 // diffusion and sidewall drag of each computational edge in edgep order.
-template <int NF>
-__global__ __launch_bounds__(256) void k_wp_source(Geo G, WPArgs A) {
-  const int t = xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
+template <int NF, bool BAND>
+__global__ __launch_bounds__(256) void k_wp_source(Geo G, WPArgs A, Bands B) {
+  const int v = xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
+  const int t = BAND ? v / B.nb : v, ka = BAND ? (v - t * B.nb) * B.len : 0, kz = BAND ? ka + B.len : 0x7fffffff;
   if (t >= G.Nt) return;
   const int s = t * 64 + l, n = G.nk[s];
-  if (n == 0) return;
+  const int ke = min(n, kz);
+  if (n == 0 || ka >= ke) return;
   const int NS = G.NS, nf = G.nf[s], ct = G.ctop[s];
   const uint32_t base = (uint32_t)(G.toff[t] + l);
   const double Ac = G.Ac[s];
@@ -163,11 +170,11 @@ __global__ __launch_bounds__(256) void k_wp_source(Geo G, WPArgs A) {
   auto Wd = [&](uint32_t b, int k) { return at32(A.w, b + (uint32_t)k * 64u); };
   // w of this column at k and k+1, and of each face's other column at k and
   // k+1 over the face's levels, slide down the column in registers
-  double wo0 = Wd(base, 0), wo1 = Wd(base, 1);
+  double wo0 = Wd(base, ka), wo1 = Wd(base, ka + 1);
   double wn0[NF], wn1[NF];
 #pragma unroll
   for (int f = 0; f < NF; f++) { wn0[f] = 0; wn1[f] = 0; }
-  for (int k = 0; k < n; k++) {
+  for (int k = ka; k < ke; k++) {
     double st = 0;
     const uint32_t kk = (uint32_t)k * 64u;
     if (adv && k >= ct) {
@@ -182,7 +189,7 @@ __global__ __launch_bounds__(256) void k_wp_source(Geo G, WPArgs A) {
       if (f >= nf || !ocomp[f]) continue;
       if (k >= okmin[f] && k < onke[f]) {
         const uint32_t other = ofirst[f] ? oc2[f] : oc1[f];
-        if (k == okmin[f]) wn0[f] = Wd(other, k);
+        if (k == okmin[f] || (BAND && k == ka)) wn0[f] = Wd(other, k);
         else wn0[f] = wn1[f];
         wn1[f] = Wd(other, k + 1);
         const double nln = at32(A.nu_lax, other + kk);
@@ -371,9 +378,14 @@ int sunhip_w_predict(sunhip_grid *g, const sunhip_wpred_params *p) {
   if (rc) return rc;
   const Geo G = g->geo();
   const int nc = (g->Nt + 3) / 4, ne = (g->Net + 3) / 4;
+  // BAND kernels: a wave per tile and band of levels (2000 columns of 50 levels:
+  // source 141 -> 24 us)
+  const Bands Bc = level_bands(g, g->Nt), Be = level_bands(g, g->Net);
+  const int ncb = (g->Nt * Bc.nb + 3) / 4;
   if (A.scheme) {
     int ps = prof_begin(g, PK_OTHER);
-    k_wp_centres<<<nc, 256, 0, g->stream>>>(G, A);
+    if (Bc.nb > 1) k_wp_centres<true><<<ncb, 256, 0, g->stream>>>(G, A, Bc);
+    else k_wp_centres<false><<<nc, 256, 0, g->stream>>>(G, A, Bc);
     prof_end(g, ps);
     HIPCHK(hipGetLastError());
     if (A.scheme == 5) {
@@ -389,13 +401,16 @@ int sunhip_w_predict(sunhip_grid *g, const sunhip_wpred_params *p) {
       if ((rc = face_scalars_launch(g, T))) return rc;
     }
     ps = prof_begin(g, PK_OTHER);
-    k_wp_faces<<<ne, 256, 0, g->stream>>>(G, A);
+    if (Be.nb > 1) k_wp_faces<true><<<(g->Net * Be.nb + 3) / 4, 256, 0, g->stream>>>(G, A, Be);
+    else k_wp_faces<false><<<ne, 256, 0, g->stream>>>(G, A, Be);
     prof_end(g, ps);
     HIPCHK(hipGetLastError());
   }
   int ps = prof_begin(g, PK_WSOURCE);
   with_nf(g->mf, [&](auto nf) {
-    k_wp_source<decltype(nf)::value><<<nc, 256, 0, g->stream>>>(G, A);
+    constexpr int NF = decltype(nf)::value;
+    if (Bc.nb > 1) k_wp_source<NF, true><<<ncb, 256, 0, g->stream>>>(G, A, Bc);
+    else k_wp_source<NF, false><<<nc, 256, 0, g->stream>>>(G, A, Bc);
     return 0;
   });
   prof_end(g, ps);
