@@ -100,10 +100,12 @@ __device__ __forceinline__ void upred_edge_tile(const Geo &G, const UPArgs &A, i
     if (k >= ne || k < kth) return 0.0;
     return 0.5 * (at32(A.w, (uint32_t)bl + (uint32_t)k * 64u) + at32(A.w, (uint32_t)bh + (uint32_t)k * 64u));
   };
-  // mean eddy and Lax-Wendroff viscosity at the face above level k (k > et)
-  auto VIS = [&](int k) {
-    return 0.25 * (C1(A.nu_tv, k - 1) + C2(A.nu_tv, k - 1) + C1(A.nu_tv, k) + C2(A.nu_tv, k) +
-                   lw * (C1(A.nu_lax, k - 1) + C2(A.nu_lax, k - 1) + C1(A.nu_lax, k) + C2(A.nu_lax, k)));
+  // mean eddy and Lax-Wendroff viscosity at the face above level k (k > et),
+  // from the two cells' values at k - 1 (m) and k
+  struct Vis { double t1, t2, l1, l2; };
+  auto VL = [&](int k) { return Vis{C1(A.nu_tv, k), C2(A.nu_tv, k), C1(A.nu_lax, k), C2(A.nu_lax, k)}; };
+  auto VIS = [&](const Vis &m, const Vis &v) {
+    return 0.25 * (m.t1 + m.t2 + v.t1 + v.t2 + lw * (m.l1 + m.l2 + v.l1 + v.l2));
   };
   const double f1 = dt * (1 - th), fm = dt * (1 - tM), ti = th * dt, ta = dt * tM;
   bool dry = false;
@@ -112,11 +114,21 @@ __device__ __forceinline__ void upred_edge_tile(const Geo &G, const UPArgs &A, i
   double h1m = 0, h2m = 0, h1k = Z1(et), h2k = Z2(et);
   double h1p = multi ? Z1(et + 1) : 0.0, h2p = multi ? Z2(et + 1) : 0.0;
   double um = 0, uk = E(A.u, et), up = multi ? E(A.u, et + 1) : 0.0;
-  double sck = 0, scp = multi ? VIS(et + 1) : 0.0;
+  Vis vp = VL(min(et + 1, kb));  // at k + 1
+  double sck = 0, scp = multi ? VIS(VL(et), vp) : 0.0;
   double dk = adv ? DW(et) : 0.0;
   double sb_above = 0, btop = 0;  // level k-1's coefficient below it; the top row's diagonal
   double bprev = 0, dprev = 0, eprev = 0, cprev = 0;
+  // the loads of the next level's right-hand side and of the window's next
+  // entries are issued at the top of a level (at clamped levels) and their
+  // values combined at its end, so none waits behind the level's divisions
+  double rhsN = E(A.utmp, et), dkN = adv ? DW(et + 1) : 0.0;
   for (int k = et; k < ne; k++) {
+    const double rhs0 = rhsN, dk1n = dkN;
+    const int k1 = min(k + 1, kb), k2 = min(k + 2, kb);
+    const double rq = E(A.utmp, k1), h1q = Z1(k2), h2q = Z2(k2), upq = E(A.u, k2);
+    const double wlq = at32(A.w, (uint32_t)bl + (uint32_t)k2 * 64u), whq = at32(A.w, (uint32_t)bh + (uint32_t)k2 * 64u);
+    const Vis vq = VL(k2);
     if (h1k == 0 && h2k == 0) dry = true;
     const double hs = h1k + h2k;
     // viscosity coefficients above (sa) and below (sb) level k
@@ -125,7 +137,7 @@ __device__ __forceinline__ void upred_edge_tile(const Geo &G, const UPArgs &A, i
     // vertical advection coefficients (thetaM)
     double sa0 = 0, sb0 = 0, sc0 = 0;
     if (adv) {
-      const double dk1 = DW(k + 1);
+      const double dk1 = dk1n;
       const double hz = 0.5 * hs;
       sa0 = (alpha * 0.5 * (dk - fabs(dk)) + 0.5 * (1 - alpha) * dk) / hz;
       sb0 = (alpha * 0.5 * (dk + fabs(dk) - dk1 + fabs(dk1)) + 0.5 * (1 - alpha) * (dk - dk1)) / hz;
@@ -133,7 +145,7 @@ __device__ __forceinline__ void upred_edge_tile(const Geo &G, const UPArgs &A, i
       dk = dk1;
     }
     // explicit viscosity and drag, then explicit vertical advection, into U***
-    double rhs = E(A.utmp, k);
+    double rhs = rhs0;
     if (multi) {
       if (k == et) {
         if (CdT == -1) rhs += f1 * (sa * -uk - (sa + sb) * uk + sb * up);
@@ -221,8 +233,11 @@ __device__ __forceinline__ void upred_edge_tile(const Geo &G, const UPArgs &A, i
     h1m = h1k; h2m = h2k; h1k = h1p; h2k = h2p;
     um = uk; uk = up;
     sck = scp;
-    if (k + 2 < ne) { h1p = Z1(k + 2); h2p = Z2(k + 2); up = E(A.u, k + 2); scp = VIS(k + 2); }
-    else { h1p = 0; h2p = 0; up = 0; scp = 0; }
+    const bool in = k + 2 < ne;
+    h1p = in ? h1q : 0; h2p = in ? h2q : 0; up = in ? upq : 0; scp = in ? VIS(vp, vq) : 0;
+    vp = vq;
+    rhsN = rq;
+    dkN = adv && in && k + 2 >= kth ? 0.5 * (wlq + whq) : 0.0;
   }
   if (dry) { A.err[0] = 1; return; }
   // substitution, bottom up; it forms the final U*** of every wet level
@@ -232,16 +247,38 @@ __device__ __forceinline__ void upred_edge_tile(const Geo &G, const UPArgs &A, i
   bool bad = un != un;
   E(A.utmp, kb) = un;
   E(A.E, kb) = en;
-  for (int k = kb - 1; k >= et; k--) {
-    const double bk = E(A.sbp, k), ck = E(A.sc, k);
-    un = E(A.utmp, k) / bk - ck * un / bk;
-    en = E(A.sep, k) / bk - ck * en / bk;
-    bad |= un != un;
-    __builtin_nontemporal_store(un, &E(A.utmp, k));
-    E(A.E, k) = en;
+  // (four rows loaded at a time)
+  for (int k0 = kb - 1; k0 >= et; k0 -= 4) {
+    double vb[4], vc[4], vu[4], ve[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int k = max(k0 - j, et);
+      vb[j] = E(A.sbp, k); vc[j] = E(A.sc, k); vu[j] = E(A.utmp, k); ve[j] = E(A.sep, k);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int k = k0 - j;
+      if (k < et) break;
+      un = vu[j] / vb[j] - vc[j] * un / vb[j];
+      en = ve[j] / vb[j] - vc[j] * en / vb[j];
+      bad |= un != un;
+      __builtin_nontemporal_store(un, &E(A.utmp, k));
+      E(A.E, k) = en;
+    }
   }
   double Dj = 0;
-  for (int k = et; k < ne; k++) Dj += E(A.E, k) * at32(A.dzf, base + (uint32_t)k * 64u);
+  for (int k0 = et; k0 < ne; k0 += 4) {
+    double ve[4], vz[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int k = min(k0 + j, kb);
+      ve[j] = E(A.E, k);
+      vz[j] = at32(A.dzf, base + (uint32_t)k * 64u);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (k0 + j < ne) Dj += ve[j] * vz[j];
+  }
   A.D[s] = Dj;
   if (bad) A.err[1] = 1;
 }

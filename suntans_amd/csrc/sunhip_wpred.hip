@@ -292,10 +292,20 @@ __global__ __launch_bounds__(256) void k_wp_column(Geo G, WPArgs A) {
   }
   double wn = R(A.wtmp, n - 1) / R(A.sc, n - 1);
   X(A.w, n - 1) = wn;
-  for (int k = n - 2; k >= ct; k--) {
-    const double cd = R(A.sc, k);
-    wn = R(A.wtmp, k) / cd - R(A.sb, k) * wn / cd;
-    X(A.w, k) = wn;
+  for (int kb = n - 2; kb >= ct; kb -= 4) {  // four rows loaded at a time
+    double vd[4], vb[4], vw[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int k = max(kb - j, ct);
+      vd[j] = R(A.sc, k); vb[j] = R(A.sb, k); vw[j] = R(A.wtmp, k);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int k = kb - j;
+      if (k < ct) break;
+      wn = vw[j] / vd[j] - vb[j] * wn / vd[j];
+      X(A.w, k) = wn;
+    }
   }
 }
 
