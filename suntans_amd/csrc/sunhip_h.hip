@@ -314,6 +314,114 @@ __global__ __launch_bounds__(HBS) void k_hsettle(CGScal *sc, const double *pin, 
   if (host && threadIdx.x == 0) *host = S;
 }
 
+// ---- the whole solve of a small grid in one block -----------------------------
+//
+// A free-surface iteration of a few thousand cells is launch latency: two
+// launches of 5.3 and 3.9 us for 2000 cells.  Here one block of 1024 threads
+// holds up to CPT cells per thread in registers (r, M^-1 r, x, p, the
+// coefficients and neighbours) and p in LDS, and iterates until done: 21
+// iterations in one launch.  The cells' arithmetic is that of
+// k_happly_it/k_hprec_it; only the grouping of the dot products differs.  A
+// launch ends after HSM_ITERS iterations at the latest and the next one goes
+// on from r, u and p in memory.
+constexpr int HSM = 1024, HSM_ITERS = 1024;
+
+// sums of NV values over the block, in every thread
+template <int NV>
+__device__ __forceinline__ void h_block_sum(const double (&v)[NV], double (*sh)[16], double (&tot)[NV]) {
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+#pragma unroll
+  for (int i = 0; i < NV; i++) {
+    const double s = wave_sum(v[i]);
+    if (l == 0) sh[i][w] = s;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NV; i++) {
+    double s = 0;
+#pragma unroll
+    for (int j = 0; j < HSM / 64; j++) s += sh[i][j];
+    tot[i] = s;
+  }
+}
+
+template <typename T, int NF, int CPT>
+__global__ __launch_bounds__(HSM) void k_hcg_block(Geo G, HVec<T, T> V, T *rb, T *ub, T *pb, CGScal *sc,
+                                                   unsigned long long *host, unsigned long long tag) {
+  __shared__ T pl[HSM * CPT];
+  __shared__ double sh1[1][16], sh2[2][16];
+  CGScal S = *sc;
+  __syncthreads();  // every thread has read sc before thread 0 writes it at the end
+  if (S.done) return;
+  bool ok[CPT];
+  T r[CPT], u[CPT], x[CPT], p[CPT], c[CPT], fc[CPT][NF];
+  int nb[CPT][NF];
+#pragma unroll
+  for (int j = 0; j < CPT; j++) {
+    const int s = threadIdx.x + j * HSM, q = s < G.NS ? s : 0;
+    ok[j] = s < G.NS && G.nk[q] > 0 && G.comp[q] == 1;
+    r[j] = rb[q]; u[j] = ub[q]; x[j] = V.x[q]; p[j] = pb[q]; c[j] = V.coef[q];
+    const int nf = G.nf[q];
+#pragma unroll
+    for (int f = 0; f < NF; f++) {
+      const int row = f < G.mf ? f : G.mf - 1;  // rows past maxfaces are not stored
+      const int n = G.nbs[row * G.NS + q];
+      nb[j][f] = ok[j] && f < nf && n >= 0 ? n : -1;
+      fc[j][f] = V.fcoef[row * G.NS + q];
+    }
+  }
+  const int pc = S.precond;
+  for (int it = 0; it < HSM_ITERS && !S.done; it++) {
+    const T mu = (T)S.mu, nu0 = (T)S.nu;
+#pragma unroll
+    for (int j = 0; j < CPT; j++) {
+      const T v0 = u[j] + mu * p[j];  // of other cells: their u, as p is 0 there
+      if (ok[j]) {
+        x[j] = x[j] + nu0 * p[j];
+        p[j] = v0;
+      }
+      pl[threadIdx.x + j * HSM] = v0;
+    }
+    __syncthreads();
+    T y[CPT];
+    double v1[1] = {0}, t1[1];
+#pragma unroll
+    for (int j = 0; j < CPT; j++) {
+      y[j] = c[j] * p[j];
+#pragma unroll
+      for (int f = 0; f < NF; f++)
+        if (nb[j][f] >= 0) y[j] -= fc[j][f] * pl[nb[j][f]];
+      if (ok[j]) v1[0] += (double)p[j] * (double)y[j];
+    }
+    h_block_sum<1>(v1, sh1, t1);
+    h_op(&S, HOP_APPLY, t1);
+    const T nu = (T)S.nu;
+    double v2[2] = {0, 0}, t2[2];
+#pragma unroll
+    for (int j = 0; j < CPT; j++) {
+      if (!ok[j]) continue;
+      r[j] = r[j] - nu * y[j];
+      u[j] = pc == 1 ? r[j] / c[j] : r[j];
+      v2[0] += (double)r[j] * (double)u[j];
+      v2[1] += (double)r[j] * (double)r[j];
+    }
+    h_block_sum<2>(v2, sh2, t2);
+    h_op(&S, HOP_ITER, t2);
+  }
+  const T nu = (T)S.nu;  // done: the last iteration's x update
+#pragma unroll
+  for (int j = 0; j < CPT; j++) {
+    const int s = threadIdx.x + j * HSM;
+    if (!ok[j]) continue;
+    V.x[s] = S.done ? x[j] + nu * p[j] : x[j];
+    if (!S.done) { rb[s] = r[j]; ub[s] = u[j]; pb[s] = p[j]; }
+  }
+  if (threadIdx.x == 0) {
+    *sc = S;
+    __hip_atomic_store(host, tag | (S.done ? 1u : 0u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
 // r -= nu*z ; rtmp = r/hcoef (hprecond=1) or r ; dots.
 template <typename T>
 __global__ __launch_bounds__(256) void k_hprec(Geo G, const T *__restrict__ coef, const T *__restrict__ z,
@@ -457,6 +565,30 @@ int h_poll(sunhip_grid *g, CGScal *sc, int &slot, bool &pending, bool *done) {
 
 template <typename T>
 int h_loop(sunhip_grid *g, const sunhip_cg_params *prm, HSolver<T> &S, int pk_a, int pk_p) {
+  // one block up to 4096 cell slots (2048 from 6 faces: registers)
+  const int cpt = (g->NS + HSM - 1) / HSM;
+  if (prm->maxiters > 0 && cpt <= (nf_class(g->mf) <= 4 ? 4 : 2)) {
+    HVec<T, T> V{};
+    V.coef = S.coef; V.fcoef = S.fcoef; V.x = S.x;
+    for (int done = 0; done < prm->maxiters; done += HSM_ITERS) {
+      const unsigned long long tag = (unsigned long long)(++g->prog_tag & 0x7fffffff) << 32;
+      const int ps = prof_begin(g, pk_a);
+      with_nf(g->mf, [&](auto nfc) {
+        constexpr int NF = decltype(nfc)::value;
+        if (cpt <= 2)
+          k_hcg_block<T, NF, 2><<<1, HSM, 0, g->stream>>>(g->geo(), V, S.r, S.rt, S.p0, S.sc, g->h_prog, tag);
+        else if constexpr (NF <= 4)
+          k_hcg_block<T, NF, 4><<<1, HSM, 0, g->stream>>>(g->geo(), V, S.r, S.rt, S.p0, S.sc, g->h_prog, tag);
+        return 0;
+      });
+      prof_end(g, ps);
+      HIPCHK(hipGetLastError());
+      if (prm->maxiters - done <= HSM_ITERS) break;
+      HIPCHK(hipStreamSynchronize(g->stream));
+      if (*(volatile unsigned long long *)g->h_prog == (tag | 1u)) break;
+    }
+    return 0;
+  }
   int every = prm->check_every > 0 ? prm->check_every : 8;
   if (every & 1) every++;
   int it = 0, rc, slot = 0;

@@ -1,0 +1,84 @@
+"""The free-surface solve of small grids in one block (up to 4096 cell slots,
+2048 from 6 faces) against the oracle, at the edges of its one, two and four
+cells per thread and on both sides of its limits: h within 1e-10 and equal
+counts; every face class; with and without the preconditioner; a solve that
+runs out of iterations, and one that goes on over several launches."""
+import numpy as np
+import pytest
+
+from suntans_amd import cases, device
+
+import _impls
+
+pytestmark = pytest.mark.gpu
+
+# cells: 64, 1024, 1026, 2048, 2050, 4096, 4100 triangles
+SIZES = [(8, 4), (32, 16), (27, 19), (32, 32), (41, 25), (64, 32), (50, 41)]
+SHAPES = {"quad": dict(planform="quad", split_every=3, nx=40, ny=40), "hex": dict(planform="hex", nx=40, ny=25),
+          "hex8": dict(planform="hex", split_every=4, maxfaces=7, nx=45, ny=40),
+          "open": dict(nx=40, ny=20, open_marks=cases.open_ends())}
+
+
+def check(st, precond=1):
+    st.set("D", cases.depth_integrated_D(st))
+    st.set_prop(hprecond=precond, epsilon=1e-10, maxiters=3000)
+    o = _impls.oracle()
+    a = st.clone()
+    h0 = st.get("h")
+    dg = device.DeviceGrid(st)
+    for f in ("D", "htmp", "h"):
+        dg.upload(f, st.get(f))
+    o.cgsolve(a)
+    g = st.get_prop
+    r = dg.h_solve(g("grav"), g("theta"), g("dt"), maxiters=3000, precond=precond, epsilon=1e-10)
+    h = dg.download("h", st.Nc)
+    assert r["converged"] and r["niters"] == o.stats("h")[0]
+    assert np.linalg.norm(h - a.get("h")) <= 1e-10 * np.linalg.norm(a.get("h"))
+    return dg, h, h0
+
+
+@pytest.mark.parametrize("nx,ny", SIZES, ids=["%dx%d" % s for s in SIZES])
+def test_sizes(gpu_available, nx, ny):
+    check(cases.tiny(nx, nx=nx, ny=ny, Nkmax=5, min_layers=1))[0].close()
+
+
+@pytest.mark.parametrize("precond", [0, 1])
+@pytest.mark.parametrize("name", sorted(SHAPES))
+def test_shapes(gpu_available, name, precond):
+    check(cases.tiny(4, Nkmax=5, min_layers=1, **SHAPES[name]), precond)[0].close()
+
+
+def test_iteration_limits(gpu_available):
+    """maxiters iterations where the tolerance is out of reach."""
+    st = cases.tiny(7, nx=20, ny=10, Nkmax=5, min_layers=1)
+    dg, h, h0 = check(st)
+    g = st.get_prop
+    for n in (0, 1, 3):
+        dg.upload("htmp", st.get("htmp"))
+        dg.upload("h", h0)
+        r = dg.h_solve(g("grav"), g("theta"), g("dt"), maxiters=n, precond=1, epsilon=1e-300)
+        assert r["niters"] == n and not r["converged"], r
+    dg.close()
+
+
+def test_several_launches(gpu_available):
+    """A stiff solve without the preconditioner (2815 iterations in the oracle,
+    1024 per launch here).  Its count is decided by rounding, which the dot
+    products' grouping changes: 5%; h agrees to 1e-8."""
+    st = cases.tiny(7, nx=64, ny=32, Nkmax=5, min_layers=1)
+    st.set("D", cases.depth_integrated_D(st) * np.random.default_rng(0).uniform(1e-3, 1, st.Ne) ** 3)
+    st.set_prop(dt=5000.0, hprecond=0, epsilon=1e-10, maxiters=9000)
+    o = _impls.oracle()
+    a = st.clone()
+    dg = device.DeviceGrid(st)
+    for f in ("D", "htmp", "h"):
+        dg.upload(f, st.get(f))
+    o.cgsolve(a)
+    n0 = o.stats("h")[0]
+    assert n0 > 2048
+    g = st.get_prop
+    r = dg.h_solve(g("grav"), g("theta"), 5000.0, maxiters=9000, precond=0, epsilon=1e-10)
+    h = dg.download("h", st.Nc)
+    dg.close()
+    assert r["converged"] and abs(r["niters"] - n0) <= 0.05 * n0
+    assert np.linalg.norm(h - a.get("h")) <= 1e-8 * np.linalg.norm(a.get("h"))
