@@ -936,8 +936,7 @@ int sunhip_batch_poll(sunhip_batch *b, int64_t *tags, int *kinds, sunhip_cg_stat
         b->dirty = true;
       } else if (t.mstate == M_INNER && c.done) {
         t.inner_total += c.iter;
-        if ((rc = q_end32(t.g, t.q32))) return rc;
-        if ((rc = q_mix_update(t.g, const_cast<double *>(t.R.vin), t.q32.x))) return rc;
+        if ((rc = q_mix_finish(t.g, const_cast<double *>(t.R.vin), t.q32, t.q32.sc))) return rc;
         t.outer++;
         t.mstate = M_RESID;
         b->dirty = true;
@@ -950,7 +949,6 @@ int sunhip_batch_poll(sunhip_batch *b, int64_t *tags, int *kinds, sunhip_cg_stat
       continue;
     }
     if (t.kind == T_Q64) rc = q_end64(t.g, t.q64);
-    else if (t.kind == T_Q32) rc = q_end32(t.g, t.q32);
     else rc = h_end64(t.g, t.h64);
     if (rc) return rc;
     if (tags) tags[out] = t.tag;
@@ -980,7 +978,7 @@ int sunhip_batch_begin_q_mixed(sunhip_batch *b, sunhip_grid *g, const sunhip_cg_
   Task t{};
   t.g = g; t.kind = T_QMIX; t.tag = tag;
   if ((t.stage = take_stage(b)) < 0) return -3;
-  if ((rc = q_mixed_prepare(g, prm, &t.q32, &t.R))) return rc;
+  if ((rc = q_mixed_prepare(g, prm, &t.q32, &t.R, q_seg_fits(g)))) return rc;
   t.mstate = M_RESID;
   t.prm = *prm;
   t.inner_tol = inner_tol;

@@ -13,8 +13,11 @@
 // kernel (a tuning choice); both add the partials in a fixed order, so a
 // solve is reproducible run to run.  Element-wise arithmetic keeps the
 // reference's operation order and is built without FMA contraction, so
-// OperatorQ and the preconditioner agree with the reference bit for bit;
-// only the summation order of the dot products differs.
+// OperatorQ and the Preconditioner entry point agree with the reference bit
+// for bit.  Inside a solve the preconditioner multiplies by inverse pivots
+// formed once, where the reference divides twice per level and application,
+// and the dot products are summed in another order.  Small and middle grids
+// run the iteration of sunhip_qseg.hip.
 //
 // The kernels are templated on the storage type T of vectors and
 // coefficients.  T=double is the drop-in; T=float is the inner solve of the
@@ -22,7 +25,7 @@
 // accumulate in double and whose outer residual, convergence test and
 // solution update stay in FP64.
 //
-// Both kernels walk a column U levels at a time (a tuning choice, 1, 2 or 4)
+// These kernels walk a column U levels at a time (a tuning choice, 1 to 8)
 // and issue every load of a group before its arithmetic, with addresses
 // clamped into the column (a tile stores one level more than its deepest
 // column), so no load waits behind a branch.
@@ -366,18 +369,13 @@ __global__ void k_cast(const TI *__restrict__ a, TO *__restrict__ b, int64_t n) 
   if (i < n) b[i] = (TO)a[i];
 }
 
-// x64 += e32 on the computational columns (mixed form, FP64 accumulation).
-__global__ __launch_bounds__(256) void k_mix_update(Geo G, double *__restrict__ x, const float *__restrict__ e) {
-  mix_update_tile(G, x, e, blockIdx.x * 4 + (threadIdx.x >> 6), threadIdx.x & 63);
-}
-
-// The inner solve's k_qfinish and k_mix_update in one launch (mixed form).
+// The inner solve's last x update and x64 += e32 in one launch (mixed form),
+// a wave per tile and band of levels.
 __global__ __launch_bounds__(256) void k_mix_finish(Geo G, double *__restrict__ x, const float *__restrict__ e,
                                                     const float *__restrict__ p0, const float *__restrict__ p1,
-                                                    const CGScal *sc) {
-  const int it = sc->iter;
-  mix_finish_tile(G, x, e, (it & 1) ? p1 : p0, (float)sc->nu, it != 0, blockIdx.x * 4 + (threadIdx.x >> 6),
-                  threadIdx.x & 63);
+                                                    const CGScal *sc, Bands B) {
+  const int it = sc->iter, v = blockIdx.x * 4 + (threadIdx.x >> 6), t = v / B.nb, k0 = (v - t * B.nb) * B.len;
+  mix_finish_tile(G, x, e, (it & 1) ? p1 : p0, (float)sc->nu, it != 0, t, threadIdx.x & 63, k0, k0 + B.len);
 }
 
 // ---------------------------------------------------------------------------
@@ -516,7 +514,7 @@ int launch_apply(sunhip_grid *g, CGScal *sc, const QVec<T, TO> &V, const Red &R,
   if constexpr (MODE == QM_FUSED && std::is_same<T, TO>::value) {
     // The exchange kernel, unless another launch shape was asked for.  With
     // few tiles the plain kernel at 2 levels per group has more waves in
-    // flight: 790 tiles of triangles 50 us against 58 (q50k), 1570 tiles 83
+    // flight: 790 tiles of triangles 50 us against 58, 1570 tiles 83
     // against 80, 3900 tiles 239 against 204; with 6 or 8 faces the exchange
     // saves most gathers at any size (1090 tiles of hexagons 114 against 86).
     // Its register budget of 4 waves per SIMD spills from 4 faces up (780
@@ -914,17 +912,13 @@ int upload_scal(sunhip_grid *g, CGScal *d, const sunhip_cg_params *prm, CGScal *
 int q_begin64(sunhip_grid *g, const sunhip_cg_params *prm, QSolver<double> *S, CGScal *stage, CGScal *sc) {
   HIPCHK(hipSetDevice(g->device));
   F64 B;
-  return q_setup(g, prm, B, *S, stage, sc);
+  const bool seg = prm->precond == 2 && q_seg_fits(g);  // the same values in three shorter launches
+  int rc = q_setup(g, prm, B, *S, stage, sc, seg);
+  return rc || !seg ? rc : q_seg_settle(g, S->sc);
 }
 
 int q_end64(sunhip_grid *g, const QSolver<double> &S) {
   k_qfinish<double><<<nb4(g), 256, 0, g->stream>>>(g->geo(), S.x, S.p0, S.p1, S.sc);
-  HIPCHK(hipGetLastError());
-  return 0;
-}
-
-int q_end32(sunhip_grid *g, const QSolver<float> &S) {
-  k_qfinish<float><<<nb4(g), 256, 0, g->stream>>>(g->geo(), S.x, S.p0, S.p1, S.sc);
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -1010,14 +1004,19 @@ int q_windows(sunhip_grid *g, const double *coef, const double *dzf, ZReg *Z) {
 
 int q_inner_begin(sunhip_grid *g, const sunhip_cg_params *inner, QSolver<float> &S32, CGScal *stage) {
   int rc;
+  if (S32.ql) {  // prepared for the kernels of sunhip_qseg.hip
+    if ((rc = seg_start<float>(g, inner, S32, nullptr, true))) return rc;
+    return q_seg_settle(g, S32.sc);
+  }
   if ((rc = upload_scal(g, S32.sc, inner, stage))) return rc;
   k_fill<float><<<(unsigned)((g->NT + 255) / 256), 256, 0, g->stream>>>(S32.x, g->NT, 0.0f);
   HIPCHK(hipGetLastError());
   return cg_start<float>(g, inner, S32);
 }
 
-int q_mix_update(sunhip_grid *g, double *x, const float *e) {
-  k_mix_update<<<nb4(g), 256, 0, g->stream>>>(g->geo(), x, e);
+int q_mix_finish(sunhip_grid *g, double *x, const QSolver<float> &S, const CGScal *sc) {
+  const Bands B = level_bands(g, g->Nt);
+  k_mix_finish<<<(g->Nt * B.nb + 3) / 4, 256, 0, g->stream>>>(g->geo(), x, S.x, S.p0, S.p1, sc, B);
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -1103,8 +1102,7 @@ int sunhip_q_solve_mixed(sunhip_grid *g, const sunhip_cg_params *prm, double inn
     const CGScal *sc = seg ? S.sc + 1 : S.sc;  // the settled scalars
     // x += e (with the inner solve's last update), the next residual, then
     // one wait for both the inner count and the residual
-    k_mix_finish<<<nb4(g), 256, 0, g->stream>>>(g->geo(), const_cast<double *>(R.vin), S.x, S.p0, S.p1, sc);
-    HIPCHK(hipGetLastError());
+    if ((rc = q_mix_finish(g, const_cast<double *>(R.vin), S, sc))) return rc;
     HIPCHK(hipMemcpyAsync(&g->h_poll[0], sc, sizeof(CGScal), hipMemcpyDeviceToHost, g->stream));
     if ((rc = residual())) return rc;
     HIPCHK(hipStreamSynchronize(g->stream));

@@ -508,8 +508,21 @@ bool q_seg_ok(const sunhip_grid *g, const sunhip_cg_params *prm) {
   // every knob of the one-lane-per-column kernels at its default
   const bool plain = g->tune_xchg < 0 && g->tune_tiles == 4 && !g->tune_blk && !g->tune_band && !g->tune_minw &&
                      g->tune_unroll == 4 && g->tune_nts && g->tune_rzid && g->tune_phead < 0 && g->tune_punroll == 8 &&
-                     g->tune_reduce == 1 && g->tune_order;
-  return plain && prm->precond == 2 && g->Nt <= SUNHIP_QSEG_TILES && seg_count(g) <= 16;
+                     g->tune_reduce == 1;
+  return plain && prm->precond == 2 && q_seg_fits(g);
+}
+
+bool q_seg_fits(const sunhip_grid *g) {
+  return g->tune_order && g->Nt <= SUNHIP_QSEG_TILES && seg_count(g) <= 16;
+}
+
+int q_seg_settle(sunhip_grid *g, CGScal *sc) {
+  // one block reads all scalars before it writes them
+  const int nb4 = (g->Nt + 3) / 4;
+  k_qend_seg<double><<<1, 256, 0, g->stream>>>(g->geo(), nullptr, nullptr, nullptr, sc, sc, g->d_part + 4 * nb4, nb4,
+                                               nullptr, 1);
+  HIPCHK(hipGetLastError());
+  return 0;
 }
 
 // Call fn<SPW> with the preconditioner's segments per wave.

@@ -1213,14 +1213,15 @@ __device__ __forceinline__ void mix_update_tile(const Geo &G, double *__restrict
 
 // The inner FP32 solve's last x update (qfinish_tile, when upd) and then
 // x64 += e32 (mix_update_tile) in one pass over tile t, with the same
-// roundings as the two passes.
+// roundings as the two passes; levels [ka, kz).
 __device__ __forceinline__ void mix_finish_tile(const Geo &G, double *__restrict__ x, const float *__restrict__ e,
-                                                const float *__restrict__ p, float nu, bool upd, int t, int l) {
+                                                const float *__restrict__ p, float nu, bool upd, int t, int l,
+                                                int ka = 0, int kz = 0x7fffffff) {
   if (t >= G.Nt) return;
-  const int s = t * 64 + l, n = G.nk[s];
-  if (n == 0 || G.comp[s] != 1) return;
+  const int s = t * 64 + l, n = min(G.nk[s], kz);
+  if (n <= ka || G.comp[s] != 1) return;
   const int64_t base = G.toff[t] + l;
-  for (int k = G.ctop[s]; k < n; k++) {
+  for (int k = max(G.ctop[s], ka); k < n; k++) {
     const int64_t idx = base + (int64_t)k * 64;
     float ek = e[idx];
     if (upd) ek = ek + nu * p[idx];

@@ -50,6 +50,10 @@ int q_windows(sunhip_grid *g, const double *coef, const double *dzf, ZReg *Z);
 // 135, every CU then having waves enough either way.
 #define SUNHIP_QSEG_TILES 1024
 bool q_seg_ok(const sunhip_grid *g, const sunhip_cg_params *prm);
+// Whether the grid's size and dispatch order allow these kernels at all.
+bool q_seg_fits(const sunhip_grid *g);
+// The scalars at sc after their pending first step (q_seg_start), in place.
+int q_seg_settle(sunhip_grid *g, CGScal *sc);
 // Coefficients, inverse pivots and l (QSolver::ql) from dzz, or the last two
 // from FP32 coefficients.
 int q_seg_setup64(sunhip_grid *g, const double *dzz, double *coef, double *bq, double *ql);
@@ -74,7 +78,6 @@ int upload_scal(sunhip_grid *g, CGScal *d, const sunhip_cg_params *prm, CGScal *
 int q_begin64(sunhip_grid *g, const sunhip_cg_params *prm, QSolver<double> *S, CGScal *stage, CGScal *sc = nullptr);
 // x += nu*p of the last iteration.
 int q_end64(sunhip_grid *g, const QSolver<double> &S);
-int q_end32(sunhip_grid *g, const QSolver<float> &S);
 
 // Mixed form: FP64 coefficients, FP32 copies of coef/dzf/D, FP32 pivots;
 // S32 gets the FP32 PCG buffers (x = the correction e, scalars g->d_ms) and
@@ -84,8 +87,8 @@ int q_mixed_prepare(sunhip_grid *g, const sunhip_cg_params *prm, QSolver<float> 
                     bool seg = false);
 // Inner FP32 PCG from e = 0 on the residual already in S32.r.
 int q_inner_begin(sunhip_grid *g, const sunhip_cg_params *inner, QSolver<float> &S32, CGScal *stage);
-// x64 += e32.
-int q_mix_update(sunhip_grid *g, double *x, const float *e);
+// The inner solve's last x update (scalars at sc), then x64 += e32.
+int q_mix_finish(sunhip_grid *g, double *x, const QSolver<float> &S, const CGScal *sc);
 
 // Free surface, FP64: coefficients, x = 0 on computational cells,
 // r = b - L x, first preconditioned residual (main/phys.c:3108-3158).

@@ -68,3 +68,49 @@ def test_shapes(gpu_available, name):
     st = cases.tiny(5, **SHAPES[name])
     same(st)
     same(st, mixed=True)
+
+
+# members up to and past the limit of 1024 tiles (65536 cells)
+MEMBERS = [SIZES[:7], SIZES[7:], [(129, 254, 9), (129, 255, 9), (2, 3, 8)]]
+
+
+@pytest.mark.parametrize("sizes", MEMBERS, ids=["shallow", "deep", "limit"])
+def test_batch_members(gpu_available, sizes):
+    """A batch starts small members with these kernels.  Each member takes
+    the solve's own iteration count within one (its sums are per tile, not per
+    group of four) to the same q within 1e-10."""
+    sts = [cases.tiny(nx + lv, nx=nx, ny=max(ny, 1), Nkmax=lv, min_layers=min(3, lv - 4)) for nx, ny, lv in sizes]
+    one, many = [], []
+    for st in sts:
+        for to in (one, many):
+            dg = device.DeviceGrid(st)
+            device.member_upload(dg, st)
+            to.append(dg)
+    b = device.Batch()
+    for again in range(2):  # the second time on used buffers
+        for st, dg, mg in zip(sts, one, many):
+            device.member_upload(dg, st)
+            device.member_upload(mg, st)
+        stats = b.q_solve(many, epsilon=1e-10)
+        for dg, mg, s in zip(one, many, stats):
+            w = dg.q_solve(epsilon=1e-10)
+            n = dg.sizes()["Nflat"]
+            qw, q = dg.download("q", n), mg.download("q", n)
+            assert s["converged"] == w["converged"] == 1 and abs(s["niters"] - w["niters"]) <= 1
+            assert np.linalg.norm(q - qw) <= 1e-10 * np.linalg.norm(qw)
+    for st, dg, mg in zip(sts, one, many):
+        device.member_upload(dg, st)
+        device.member_upload(mg, st)
+    # mixed: both end below a residual of 1e-10, so q is within 1e-8 (the
+    # bound of the mixed form's other tests)
+    stats = b.q_solve_mixed(many, epsilon=1e-10, inner_tol=1e-4)
+    for dg, mg, s in zip(one, many, stats):
+        w = dg.q_solve_mixed(epsilon=1e-10, inner_tol=1e-4)
+        n = dg.sizes()["Nflat"]
+        qw, q = dg.download("q", n), mg.download("q", n)
+        assert s["converged"] == 1 and s["niters"] == w["niters"]
+        assert abs(s["inner_iters"] - w["inner_iters"]) <= s["niters"]
+        assert np.linalg.norm(q - qw) <= 1e-8 * np.linalg.norm(qw)
+    for dg in one + many:
+        dg.close()
+    b.close()
