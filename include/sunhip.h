@@ -63,7 +63,9 @@ typedef struct {
   int precond;         /* qprecond (0 none, 2 vertical line) or hprecond (0/1) */
   int resnorm;
   double epsilon;      /* qepsilon or epsilon */
-  int check_every;     /* iterations between host convergence polls (0: auto) */
+  int check_every;     /* iterations between host convergence polls (0: auto); the
+                          pressure solve of a small grid and the free-surface solve of
+                          at most 4096 cells follow the device without polls */
   int qc_alias;        /* qprecond=1 only: 1 when the caller's c rows are its residual rows, as in
                           Solve (main/phys.c:1280 passes phys->stmp3, CGSolveQ's r), so the final
                           x /= c divides by the final residual (main/phys.c:2539-2546); 0 divides
@@ -181,8 +183,9 @@ int sunhip_q_coefficients(sunhip_grid *g);
  * order), "xchg" (the iteration's operator kernel exchanges neighbour values
  * inside each wave through LDS, gathering only cross-tile neighbours from
  * memory: 0 off, 1 on, 2 on with a register budget of 4 waves per SIMD, 3 on
- * with 2 levels per load group, 4-6 the pipelined form; -1, the default: 2
- * from 4096 tiles up, else 0), "tvd_group" (levels per load group of the
+ * with 2 levels per load group, 4-6 the pipelined form; -1, the default: 0
+ * below 1536 tiles of cells of at most 4 faces, else 2 for triangles and 1
+ * for cells of more faces), "tvd_group" (levels per load group of the
  * scalar step's column update: 1, 2 (the default) or 4), "prec_lds" (levels
  * below the preconditioner's register head of 16 or 24 that keep their
  * Thomas rows in LDS between the sweeps: 0 or 12, the default), "tvd_head" (Thomas
@@ -194,7 +197,9 @@ int sunhip_q_coefficients(sunhip_grid *g);
  * others' sums: 256, 512, 1024 (the default) or 2048).  Only "tiles",
  * "reduce", "rzid", "band", "order" and "h_blocks" change the rounding of a
  * dot product;
- * every other knob gives bit-identical results. */
+ * every other knob gives bit-identical results.  A pressure solve on at most
+ * 1024 tiles with every operator and preconditioner knob at its default runs
+ * kernels of its own (a block per tile), with the same results. */
 int sunhip_set_tuning(sunhip_grid *g, const char *key, int value);
 /* Per-kernel device time: sunhip_profile(g, 1) starts recording an event
  * pair around every solver kernel launch; sunhip_kernel_times fills ms[] and

@@ -15,8 +15,8 @@
 using namespace sunhip;
 
 // BAND: a wave per tile and band of levels (Bands), else one per tile.  The
-// lock exchange (32 tiles of 50 levels): source 51 -> 10 us, Corrector 54 -> 9,
-// Continuity 70 -> 17.
+// lock exchange (32 tiles of 50 levels): source 12.6 us, Corrector 53 -> 12.8,
+// Continuity 70 -> 17.8.
 template <int NF, bool BAND>
 __global__ __launch_bounds__(256) void k_qsource(Geo G, StepArgs A, Bands B) {
   const int v = xcd_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;

@@ -389,7 +389,7 @@ int sunhip_w_predict(sunhip_grid *g, const sunhip_wpred_params *p) {
   const Geo G = g->geo();
   const int nc = (g->Nt + 3) / 4, ne = (g->Net + 3) / 4;
   // BAND kernels: a wave per tile and band of levels (2000 columns of 50 levels:
-  // source 141 -> 24 us)
+  // source 143 -> 27 us)
   const Bands Bc = level_bands(g, g->Nt), Be = level_bands(g, g->Net);
   const int ncb = (g->Nt * Bc.nb + 3) / 4;
   if (A.scheme) {
