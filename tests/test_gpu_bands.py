@@ -60,3 +60,47 @@ def test_stencils_and_predictors(gpu_available, levels, planform):
     b = st.clone()
     d.set_flux_height(b)
     assert np.array_equal(b.get("dzf"), want)
+
+
+@pytest.mark.parametrize("planform", ["tri", "quad", "hex"])
+def test_batch_stencils_and_scalars(gpu_available, planform):
+    """The same passes over a batch of grids of all these depths, and the TVD
+    face passes, against the oracle bit for bit."""
+    o = _impls.oracle()
+    sts = [grid(levels, planform=planform) for levels in LEVELS]
+    th, dt = sts[0].get_prop("theta"), sts[0].get_prop("dt")
+    step, scal = [], []
+    for i, st in enumerate(sts):
+        rng = np.random.default_rng(i)
+        st.set("qc", rng.normal(size=st.get("qc").shape))
+        st.set("q", rng.normal(size=st.get("q").shape))
+        st.set_prop(TVDsalt=3 + i % 2, n=2)
+        dg = device.DeviceGrid(st)
+        device.member_upload_step(dg, st)
+        dg.upload("q", st.get("qc"))
+        step.append(dg)
+        dg = device.DeviceGrid(st)
+        device.member_upload_tvd(dg, st)
+        scal.append(dg)
+    b = device.Batch()
+    b.compute_qsource(step, th, dt)
+    b.correct(step, th, dt)
+    b.update_scalars(scal, [(st.get_prop("theta"), st.get_prop("dt"), st.get_prop("kappa_s"), 3 + i % 2, 2)
+                            for i, st in enumerate(sts)])
+    b.sync()
+    for st, dg, sg in zip(sts, step, scal):
+        m = st.wet_mask()
+        a = st.clone()
+        o.update_salinity(a)
+        assert np.array_equal(sg.download("s", len(m))[m], a.get("s")[m])
+        a = st.clone()
+        a.set_prop(theta=th, dt=dt)
+        o.compute_qsource(a)
+        assert np.array_equal(dg.download("src", len(m))[m], a.get("stmp")[m])
+        o.corrector(a)
+        o.continuity(a)
+        for f, g in (("qp", "q"), ("w", "w"), ("u", "u")):
+            assert np.array_equal(dg.download(f, len(a.get(g))), a.get(g)), f
+        dg.close()
+        sg.close()
+    b.close()
