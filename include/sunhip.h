@@ -194,12 +194,19 @@ int sunhip_q_coefficients(sunhip_grid *g);
  * "tvd_sums_group" (the same as "tvd_group" for the TVD inflow sums: 1, 2 or
  * 4, the default), "h_blocks"
  * (most blocks of the free-surface iteration kernels, each adding all the
- * others' sums: 256, 512, 1024 (the default) or 2048).  Only "tiles",
- * "reduce", "rzid", "band", "order" and "h_blocks" change the rounding of a
- * dot product;
- * every other knob gives bit-identical results.  A pressure solve on at most
- * 1024 tiles with every operator and preconditioner knob at its default runs
- * kernels of its own (a block per tile), with the same results. */
+ * others' sums: 256, 512, 1024 (the default) or 2048; no effect up to 4096
+ * cells, which one block solves), "small" (1, the default: small grids run
+ * kernels of their own -- pressure iteration and scalar column update with a
+ * block per tile, stencils and predictors by bands of levels, the free
+ * surface in one block; 0: the kernels of large grids at every size; in a
+ * batch call 0 for all members if it is 0 for one).  Only "tiles", "reduce",
+ * "rzid", "band", "order" and "h_blocks", and "small" in the free-surface
+ * solve, change the rounding of a dot product; every other knob gives
+ * bit-identical results.  The pressure iteration of small grids takes every
+ * operator and preconditioner knob ("unroll", "prec_unroll", "reduce",
+ * "tiles", "ntstore", "rzid", "minwaves", "blocklds", "band", "prec_head",
+ * "order", "xchg") at its default: setting one of them selects the kernels of
+ * large grids, which it then shapes.  "zreg" has no effect on it. */
 int sunhip_set_tuning(sunhip_grid *g, const char *key, int value);
 /* Per-kernel device time: sunhip_profile(g, 1) starts recording an event
  * pair around every solver kernel launch; sunhip_kernel_times fills ms[] and

@@ -225,8 +225,8 @@ __global__ void kb_gather(CGScal *const *__restrict__ src, CGScal *__restrict__ 
 // Whole columns against bands and segments, calls over 12 members: 20,800
 // items source 746 / 730 us, Corrector and Continuity 1890 / 2072, scalar step
 // 2722 / 2662; 47,000 items 1517 / 1607, 3630 / 4628, 5600 / 5423.
-static Bands batch_bands(int items, int depth) {
-  if (items > 16384) return Bands{1, 0x3fffffff};
+static Bands batch_bands(int items, int depth, bool small) {
+  if (items > 16384 || !small) return Bands{1, 0x3fffffff};
   return Bands{(depth + 1 + 31) / 32, 32};
 }
 
@@ -1150,8 +1150,13 @@ int sunhip_batch_update_scalars(sunhip_batch *b, sunhip_grid **gs, int n, const 
   // copy (the order of sunhip_update_scalars)
   int mf = 3;
   int depth = 0;
-  for (int i = 0; i < n; i++) mf = std::max(mf, gs[i]->mf), depth = std::max(depth, gs[i]->maxdepth);
-  const Bands Bc = batch_bands(nc, depth), Be = batch_bands(ne, depth);
+  bool small = true;  // "small" of every member
+  for (int i = 0; i < n; i++) {
+    mf = std::max(mf, gs[i]->mf);
+    depth = std::max(depth, gs[i]->maxdepth);
+    small &= gs[i]->tune_small != 0;
+  }
+  const Bands Bc = batch_bands(nc, depth, small), Be = batch_bands(ne, depth, small);
   with_nf(mf, [&](auto nf) {
     kb_tvd_sums<decltype(nf)::value><<<dim3((nc + BW - 1) / BW, Bc.nb), 256, 0, b->stream>>>(b->ttvd.d, b->wtc.d, nc,
                                                                                              Bc.len);
@@ -1175,12 +1180,13 @@ int sunhip_batch_update_scalars(sunhip_batch *b, sunhip_grid **gs, int n, const 
 // Member table and work list of a stencil launch; returns the number of work
 // items (0: nothing to launch) or a negative error.
 static int step_tables(sunhip_batch *b, sunhip_grid **gs, int n, const double *theta, const double *dt,
-                       const char *qc, const char *q, const char *w, const char *src, int *mf, int *depth) {
+                       const char *qc, const char *q, const char *w, const char *src, int *mf, int *depth, bool *small) {
   int rc;
   std::vector<BSMember> tab(n);
   std::vector<int2> wk;
   *mf = 3;
   *depth = 0;
+  *small = true;
   for (int i = 0; i < n; i++) {
     sunhip_grid *g = gs[i];
     if ((rc = sunhip_batch_attach(b, g))) return rc;
@@ -1189,6 +1195,7 @@ static int step_tables(sunhip_batch *b, sunhip_grid **gs, int n, const double *t
     for (int t = 0; t < std::max(g->Nt, g->Net); t++) wk.push_back(make_int2(i, t));
     *mf = std::max(*mf, g->mf);
     *depth = std::max(*depth, g->maxdepth);
+    *small &= g->tune_small != 0;
   }
   if (n == 0) return 0;
   HIPCHK(hipStreamSynchronize(b->stream));  // the staging area is reused
@@ -1206,9 +1213,10 @@ int sunhip_batch_compute_qsource(sunhip_batch *b, sunhip_grid **gs, int n, const
                                  const char *src) {
   HIPCHK(hipSetDevice(b->device));
   int mf, depth;
-  const int nw = step_tables(b, gs, n, theta, dt, "q", "qp", "w", src, &mf, &depth);
+  bool small;
+  const int nw = step_tables(b, gs, n, theta, dt, "q", "qp", "w", src, &mf, &depth, &small);
   if (nw <= 0) return nw;
-  const Bands B = batch_bands(nw, depth);
+  const Bands B = batch_bands(nw, depth, small);
   with_nf(mf, [&](auto nf) {
     kb_qsource<decltype(nf)::value><<<dim3((nw + BW - 1) / BW, B.nb), 256, 0, b->stream>>>(b->tstep.d, b->wstep.d, nw,
                                                                                            B.len);
@@ -1222,15 +1230,16 @@ int sunhip_batch_correct(sunhip_batch *b, sunhip_grid **gs, int n, const double 
                          const char *qc, const char *q, const char *w) {
   HIPCHK(hipSetDevice(b->device));
   int mf, depth;
-  const int nw = step_tables(b, gs, n, theta, dt, qc, q, w, "src", &mf, &depth);
+  bool small;
+  const int nw = step_tables(b, gs, n, theta, dt, qc, q, w, "src", &mf, &depth, &small);
   if (nw <= 0) return nw;
-  const Bands B = batch_bands(nw, depth);
+  const Bands B = batch_bands(nw, depth, small);
   kb_corrector<<<dim3((nw + BW - 1) / BW, B.nb), 256, 0, b->stream>>>(b->tstep.d, b->wstep.d, nw, B.len);
   const int ns = (depth + SUNHIP_SEG - 1) / SUNHIP_SEG;
   with_nf(mf, [&](auto nf) {
     constexpr int NF = decltype(nf)::value;
     if constexpr (NF <= 4)
-      if (nw <= 16384 && ns <= 16) {
+      if (small && nw <= 16384 && ns <= 16) {
         kb_continuity_seg<NF><<<nw, ns * 64, 0, b->stream>>>(b->tstep.d, b->wstep.d);
         return 0;
       }

@@ -567,7 +567,7 @@ template <typename T>
 int h_loop(sunhip_grid *g, const sunhip_cg_params *prm, HSolver<T> &S, int pk_a, int pk_p) {
   // one block up to 4096 cell slots (2048 from 6 faces: registers)
   const int cpt = (g->NS + HSM - 1) / HSM;
-  if (prm->maxiters > 0 && cpt <= (nf_class(g->mf) <= 4 ? 4 : 2)) {
+  if (g->tune_small && prm->maxiters > 0 && cpt <= (nf_class(g->mf) <= 4 ? 4 : 2)) {
     HVec<T, T> V{};
     V.coef = S.coef; V.fcoef = S.fcoef; V.x = S.x;
     for (int done = 0; done < prm->maxiters; done += HSM_ITERS) {

@@ -135,6 +135,7 @@ struct sunhip_grid {
   int *d_b4perm = nullptr;          // depth-first dispatch order of 4-tile blocks (Geo)
   int *d_b4inv = nullptr;           // its inverse (Geo)
   int tune_order = 1;               // 1: use it
+  int tune_small = 1;               // 1: small grids run kernels of their own (segments, bands, one block)
   int tune_tvdgrp = 2;              // levels per load group of the scalar column update (1, 2, 4)
   int tune_plds = 12;               // levels below a register head of 16 or 24 kept in LDS (0, 12)
   int tune_tvdhead = 8;             // rows of the scalar column update kept in registers (0, 8, 16)
@@ -268,7 +269,7 @@ inline Bands level_bands(const sunhip_grid *g, int tiles) {
   const int most = (g->maxdepth + 1 + 7) / 8;  // w-type levels too
   int nb = tiles > 0 ? (4096 + tiles - 1) / tiles : 1;
   nb = nb < 1 ? 1 : nb > most ? most : nb;
-  if (nb <= 1) return Bands{1, 0x3fffffff};
+  if (nb <= 1 || !g->tune_small) return Bands{1, 0x3fffffff};
   const int len = ((g->maxdepth + 1 + nb - 1) / nb + 7) / 8 * 8;
   return Bands{(g->maxdepth + 1 + len - 1) / len, len};
 }

@@ -1193,6 +1193,7 @@ int sunhip_set_tuning(sunhip_grid *g, const char *key, int value) {
     if (value < -1 || value > 6) { set_error("xchg must be -1..6"); return -1; }
     g->tune_xchg = value;
   }
+  else if (!strcmp(key, "small")) g->tune_small = value != 0;
   else if (!strcmp(key, "zreg")) g->tune_zreg = value != 0;
   else if (!strcmp(key, "order")) g->tune_order = value != 0;
   else if (!strcmp(key, "tvd_group")) {

@@ -513,7 +513,7 @@ bool q_seg_ok(const sunhip_grid *g, const sunhip_cg_params *prm) {
 }
 
 bool q_seg_fits(const sunhip_grid *g) {
-  return g->tune_order && g->Nt <= SUNHIP_QSEG_TILES && seg_count(g) <= 16;
+  return g->tune_small && g->tune_order && g->Nt <= SUNHIP_QSEG_TILES && seg_count(g) <= 16;
 }
 
 int q_seg_settle(sunhip_grid *g, CGScal *sc) {

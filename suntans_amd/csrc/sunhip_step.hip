@@ -122,7 +122,7 @@ int sunhip_continuity(sunhip_grid *g, double theta, const char *w) {
   with_nf(g->mf, [&](auto nf) {
     constexpr int NF = decltype(nf)::value;
     if constexpr (NF <= 4)
-      if (g->Nt <= 1024 && ns <= 16) {
+      if (g->tune_small && g->Nt <= 1024 && ns <= 16) {
         k_continuity_seg<NF><<<g->Nt, ns * 64, 0, g->stream>>>(G, A);
         return 0;
       }

@@ -53,7 +53,7 @@ __global__ __launch_bounds__(256) void k_tvd_faces(Geo G, TvdArgs A, Bands B) {
 // here and spills from 6 faces too; 129 tiles of quadrilaterals 65 -> 40 us.
 template <int NF>
 static bool tvd_seg(const sunhip_grid *g, bool pre) {
-  if (g->tune_tvdgrp != 2 || g->tune_tvdhead != 8 || (!pre && NF > 4)) return false;
+  if (!g->tune_small || g->tune_tvdgrp != 2 || g->tune_tvdhead != 8 || (!pre && NF > 4)) return false;
   return g->maxdepth <= 8 * SUNHIP_SEG ? g->Nt <= 768 : NF <= 4 && g->maxdepth <= 16 * SUNHIP_SEG && g->Nt <= 512;
 }
 template <int NF, bool PRE, int SPW>
