@@ -151,8 +151,9 @@ __device__ __forceinline__ void tvd_faces_tile(const Geo &G, const TvdArgs &A, i
   if (t >= G.Net) return;
   const int s = t * 64 + l, ec = G.e_comp[s];
   const int64_t base = G.eoff[t] + l;
+  // etop may lie below the bottom face (Nke): the levels down to it are zeroed too
   const int nke = min(G.e_nke[s], kz), et = min(G.e_etop[s], kz);
-  if (nke <= ka) return;
+  if (max(nke, et) <= ka) return;
   const double th = A.theta;
   const bool terms = A.P1 != nullptr;
   double c1 = 0, c2 = 0;

@@ -1,0 +1,50 @@
+"""Vertical extents that the validation accepts and a moving surface does not
+produce by itself: edges whose etop lies below their bottom face."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from suntans_amd import cases, device
+
+import _impls
+
+pytestmark = pytest.mark.gpu
+
+
+def grid(levels):
+    return cases.tiny(levels, nx=13, ny=11, Nkmax=levels)
+
+
+def set_extents(dg, st, **arrays):
+    X, keep = device.extents(st, arrays)
+    device.check(device.lib().sunhip_set_extents(dg.h, C.byref(X)), "sunhip_set_extents")
+
+
+@pytest.mark.parametrize("small", [1, 0])
+@pytest.mark.parametrize("levels", [8, 17, 40, 100])
+def test_face_values_above_a_low_etop(gpu_available, levels, small):
+    """HorizontalFaceScalars zeroes the face values of every level above
+    etop (main/tvd.c:70-71, 106-107), also those below the bottom face Nke."""
+    st = grid(levels)
+    rng = np.random.default_rng(levels)
+    nke, nkc, etop = st.ints("Nke"), st.ints("Nkc"), st.ints("etop")
+    low = (nke < nkc) & (rng.random(st.Ne) < 0.7)
+    etop[low] = rng.integers(nke[low], nkc[low])
+    assert (etop > nke).any()
+    st.set_ints("etop", etop)
+    ne = len(st.get("u"))
+    before = rng.uniform(1, 2, ne)
+    dg = device.DeviceGrid(st)
+    dg.tune("small", small)
+    for f in ("s", "u", "utmp2", "dzf"):
+        dg.upload(f, st.get(f))
+    for f in ("SfHp", "SfHm"):
+        dg.upload(f, before)
+        st.set(f, before)
+    P = device.ScalarParams(st.get_prop("theta"), st.get_prop("dt"), 0.0, 4, 2, 0, 0)
+    device.check(device.lib().sunhip_face_scalars(dg.h, C.byref(P), b"s"), "sunhip_face_scalars")
+    _impls.oracle().face_scalars(st, 4)
+    for f in ("SfHp", "SfHm"):
+        assert np.array_equal(dg.download(f, ne), st.get(f)), f
+    dg.close()
