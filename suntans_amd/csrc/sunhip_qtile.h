@@ -1132,7 +1132,7 @@ __device__ __forceinline__ void qprec_ref_tile(const Geo &G, const double *__res
                                                double *__restrict__ bq, int t, int l) {
   if (t >= G.Nt) return;
   const int s = t * 64 + l, n = G.nk[s], kt = G.ctop[s];
-  if (n == 0 || G.comp[s] != 1) return;
+  if (kt >= n || G.comp[s] != 1) return;  // padding, or no wet level
   const uint32_t base = (uint32_t)(G.toff[t] + l);
   if (kt == n - 1) {
     const uint32_t idx = base + (uint32_t)kt * 64u;

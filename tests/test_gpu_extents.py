@@ -1,5 +1,6 @@
 """Vertical extents that the validation accepts and a moving surface does not
-produce by itself: edges whose etop lies below their bottom face."""
+produce by itself: edges whose etop lies below their bottom face, columns
+without a wet level."""
 import ctypes as C
 
 import numpy as np
@@ -48,3 +49,27 @@ def test_face_values_above_a_low_etop(gpu_available, levels, small):
     for f in ("SfHp", "SfHm"):
         assert np.array_equal(dg.download(f, ne), st.get(f)), f
     dg.close()
+
+
+@pytest.mark.parametrize("levels", [8, 40])
+def test_precondition_without_wet_levels(gpu_available, levels):
+    """Preconditioner leaves the rows of a column with ctop = Nk (no wet
+    level) as they are; the other columns get what they get beside columns
+    of one layer (bitwise: a column's rows depend on that column alone)."""
+    st = grid(levels)
+    n, rng = len(st.get("dzz")), np.random.default_rng(levels)
+    coef, x, xc = rng.uniform(0.5, 2, n), rng.normal(size=n), rng.normal(size=n)
+    dry = rng.random(st.Nc) < 0.3
+    out = []
+    for shift in (0, 1):  # those columns dry, or of one layer
+        dg = device.DeviceGrid(st)
+        top = np.where(dry, st.ints("Nk") - shift, st.ints("ctop"))
+        set_extents(dg, st, ctop=top, ctopold=top)
+        for f, v in (("coef", coef), ("src", x), ("q", xc)):
+            dg.upload(f, v)
+        device.check(device.lib().sunhip_q_precondition(dg.h, b"src", b"q"), "sunhip_q_precondition")
+        out.append(dg.download("q", n))
+        dg.close()
+    m = dry[st.cell_layers()[0]]
+    assert m.any() and np.array_equal(out[0][m], xc[m])
+    assert np.array_equal(out[0][~m], out[1][~m]) and not np.array_equal(out[0][~m], xc[~m])
