@@ -215,10 +215,12 @@ __global__ __launch_bounds__(256) void k_qprec(Geo G, const T *__restrict__ coef
   reduce_out<2, 256>(v, R, sc);
 }
 
+template <int KR>
 __global__ __launch_bounds__(256) void k_qprec_ref(Geo G, const double *__restrict__ coef,
                                                    const double *__restrict__ r, double *__restrict__ out,
                                                    double *__restrict__ bq) {
-  qprec_ref_tile(G, coef, r, out, bq, blockIdx.x * 4 + (threadIdx.x >> 6), threadIdx.x & 63);
+  qprec_ref_tile<KR>(G, coef, r, out, bq, tile_group(G, blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6),
+                     threadIdx.x & 63);
 }
 
 // qprecond=0: r -= nu*z, rtmp = r, alpha = eps = r.r (main/phys.c:2505-2519).
@@ -1167,7 +1169,8 @@ int sunhip_q_precondition(sunhip_grid *g, const char *x, const char *xc) {
   Field *fx, *fxc, *coef, *bq;
   int rc = field(g, x, &fx) | field(g, xc, &fxc) | field(g, "coef", &coef) | field(g, "qbp", &bq);
   if (rc) return rc;
-  k_qprec_ref<<<nb4(g), 256, 0, g->stream>>>(g->geo(), coef->d, fx->d, fxc->d, bq->d);
+  if (g->Nt >= 1024) k_qprec_ref<24><<<nb4(g), 256, 0, g->stream>>>(g->geo(), coef->d, fx->d, fxc->d, bq->d);
+  else k_qprec_ref<0><<<nb4(g), 256, 0, g->stream>>>(g->geo(), coef->d, fx->d, fxc->d, bq->d);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(g->stream));
   return 0;

@@ -1126,7 +1126,15 @@ __device__ __forceinline__ void qprec_tile(const Geo &G, const T *__restrict__ c
 }
 
 // Preconditioner as the reference orders it (main/phys.c:3577-3619 with
-// TriSolve): out = M^-1 r, bit for bit; the pivots b' go through bq.
+// TriSolve): out = M^-1 r, bit for bit.  The top KR levels keep their pivots
+// b', d' and c in registers between the sweeps; the levels below go through
+// bq (b'), out (d') and coef.  The order of operations is the same for every
+// KR.  A call, KR = 24 against one level at a time with every row through
+// memory: 1250 tiles of up to 60 levels 74 us against 160, 5000 of 40 levels
+// 146 / 414, 7800 of 100 levels 990 / 1845 (32 and 40 rows 868 and 775 there,
+// but 54 and 56 / 48 at 1950 tiles of 40); below 1024 tiles KR = 0, 300 tiles
+// of 100 levels 88 / 115.
+template <int KR>
 __device__ __forceinline__ void qprec_ref_tile(const Geo &G, const double *__restrict__ coef,
                                                const double *__restrict__ r, double *__restrict__ out,
                                                double *__restrict__ bq, int t, int l) {
@@ -1139,31 +1147,78 @@ __device__ __forceinline__ void qprec_ref_tile(const Geo &G, const double *__res
     at32(out, idx) = -0.5 * at32(r, idx) / at32(coef, idx);
     return;
   }
+  // eight levels' loads at a time (clamped to the tile's extra level), then
+  // their divisions, so the sweeps wait once per group
+  constexpr int U = 8, KH = KR > 0 ? KR : 1;
+  static_assert(KR % U == 0, "the register head is whole load groups");
+  double hb[KH], hd[KH], hc[KH];
   double cprev = 0, bprev = 1, dprev = 0;
-  double ck = at32(coef, base + (uint32_t)kt * 64u);
-  for (int k = kt; k < n; k++) {
-    const uint32_t idx = base + (uint32_t)k * 64u;
-    const double ck1 = k < n - 1 ? at32(coef, idx + 64u) : 0.0;
-    double a = 0, b, c = 0, d = at32(r, idx);
-    if (k == kt) { b = -2 * ck - ck1; c = ck1; }
-    else if (k == n - 1) { a = ck; b = -ck; }
-    else { a = ck; b = -ck - ck1; c = ck1; }
-    if (k > kt) {
-      b -= a * cprev / bprev;
-      d -= a * dprev / bprev;
+  auto group = [&](int kb, auto &&put) {
+    double c[U + 1], rv[U];
+#pragma unroll
+    for (int j = 0; j <= U; j++) {
+      const uint32_t idx = base + (uint32_t)min(kb + j, n) * 64u;
+      c[j] = at32(coef, idx);
+      if (j < U) rv[j] = at32(r, idx);
     }
-    at32(bq, idx) = b;
-    at32(out, idx) = d;
-    cprev = c; bprev = b; dprev = d; ck = ck1;
+#pragma unroll
+    for (int j = 0; j < U; j++) {
+      const int k = kb + j;
+      if (k >= n) break;
+      const double ck = c[j], ck1 = k < n - 1 ? c[j + 1] : 0.0;
+      double a = 0, b, cc = 0, d = rv[j];
+      if (k == kt) { b = -2 * ck - ck1; cc = ck1; }
+      else if (k == n - 1) { a = ck; b = -ck; }
+      else { a = ck; b = -ck - ck1; cc = ck1; }
+      if (k > kt) {
+        b -= a * cprev / bprev;
+        d -= a * dprev / bprev;
+      }
+      put(j, k, b, d, cc);
+      cprev = cc; bprev = b; dprev = d;
+    }
+  };
+  if constexpr (KR > 0) {
+#pragma unroll
+    for (int g = 0; g < KR; g += U) {
+      if (kt + g >= n) break;
+      group(kt + g, [&](int j, int, double b, double d, double c) { hb[g + j] = b; hd[g + j] = d; hc[g + j] = c; });
+    }
   }
-  double un = dprev / bprev, cn = at32(coef, base + (uint32_t)(n - 1) * 64u);
+  const int klo = kt + KR;  // first level below the head
+  for (int kb = klo; kb < n; kb += U)
+    group(kb, [&](int, int k, double b, double d, double) {
+      at32(bq, base + (uint32_t)k * 64u) = b;
+      at32(out, base + (uint32_t)k * 64u) = d;
+    });
+  double un = dprev / bprev;  // of the bottom level
   at32(out, base + (uint32_t)(n - 1) * 64u) = un;
-  for (int k = n - 2; k >= kt; k--) {
-    const uint32_t idx = base + (uint32_t)k * 64u;
-    const double b = at32(bq, idx);
-    un = at32(out, idx) / b - cn * un / b;
-    at32(out, idx) = un;
-    cn = at32(coef, idx);  // c at level k-1 is coef[k]
+  for (int ke = n - 2; ke >= klo; ke -= U) {
+    double bv[U], dv[U], cv[U];
+#pragma unroll
+    for (int j = 0; j < U; j++) {
+      const uint32_t idx = base + (uint32_t)max(ke - j, klo) * 64u;
+      bv[j] = at32(bq, idx);
+      dv[j] = at32(out, idx);
+      cv[j] = at32(coef, idx + 64u);  // c at level k is coef[k + 1]
+    }
+#pragma unroll
+    for (int j = 0; j < U; j++) {
+      const int k = ke - j;
+      if (k < klo) break;
+      un = dv[j] / bv[j] - cv[j] * un / bv[j];
+      at32(out, base + (uint32_t)k * 64u) = un;
+    }
+  }
+  if constexpr (KR > 0) {
+#pragma unroll
+    for (int j = KR - 1; j >= 0; j--) {
+      const int k = kt + j;
+      if (k < n - 1) {
+        un = hd[j] / hb[j] - hc[j] * un / hb[j];
+        at32(out, base + (uint32_t)k * 64u) = un;
+      }
+    }
   }
 }
 

@@ -9,6 +9,8 @@ import pytest
 
 from suntans_amd import cases, device
 
+import _impls
+
 pytestmark = pytest.mark.gpu
 
 
@@ -66,3 +68,22 @@ def test_default_kernels_above_1024_tiles(gpu_available, kw):
         dg.close()
     assert out[0][0] == out[1][0] and out[0][2] == out[1][2]
     assert np.array_equal(out[0][1], out[1][1]) and np.array_equal(out[0][3], out[1][3])
+
+
+@pytest.mark.parametrize("levels", [23, 24, 25, 33, 50])
+def test_entry_above_1024_tiles(gpu_available, levels):
+    """The Preconditioner entry with its 24-row register head (1024 tiles and
+    more) against the oracle, bit for bit, at columns that end around the head
+    and its load groups."""
+    st = cases.tiny(levels, nx=190, ny=180, Nkmax=levels, min_layers=min(20, levels - 4))
+    assert (st.Nc + 63) // 64 > 1024
+    rng = np.random.default_rng(levels)
+    n = len(st.get("dzz"))
+    st.set("wtmp", rng.uniform(0.5, 2, len(st.get("wtmp"))))
+    st.set("stmp", rng.normal(size=n))
+    st.set("uold", 0.0)
+    b = st.clone()
+    _impls.oracle().preconditioner(st)
+    _impls.dropin().preconditioner(b)
+    m = st.wet_mask()
+    assert np.array_equal(b.get("uold")[m], st.get("uold")[m])
