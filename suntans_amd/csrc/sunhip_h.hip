@@ -352,7 +352,10 @@ __global__ __launch_bounds__(HSM) void k_hcg_block(Geo G, HVec<T, T> V, T *rb, T
   __shared__ double sh1[1][16], sh2[2][16];
   CGScal S = *sc;
   __syncthreads();  // every thread has read sc before thread 0 writes it at the end
-  if (S.done) return;
+  if (S.done) {  // before the first iteration (a zero residual)
+    if (threadIdx.x == 0) __hip_atomic_store(host, tag | 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    return;
+  }
   bool ok[CPT];
   T r[CPT], u[CPT], x[CPT], p[CPT], c[CPT], fc[CPT][NF];
   int nb[CPT][NF];

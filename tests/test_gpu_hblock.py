@@ -82,3 +82,22 @@ def test_several_launches(gpu_available):
     dg.close()
     assert r["converged"] and abs(r["niters"] - n0) <= 0.05 * n0
     assert np.linalg.norm(h - a.get("h")) <= 1e-8 * np.linalg.norm(a.get("h"))
+
+
+def test_already_converged(gpu_available):
+    """A surface at rest without a source: the residual is zero before the
+    first iteration, and one launch reports it however many are allowed."""
+    st = cases.tiny(7, nx=20, ny=10, Nkmax=5, min_layers=1)
+    dg = device.DeviceGrid(st)
+    dg.upload("D", cases.depth_integrated_D(st))
+    g = st.get_prop
+    dg.profile(True)
+    for maxiters in (1, 1024, 1025, 200000):
+        dg.upload("htmp", np.zeros(st.Nc))
+        dg.upload("h", np.zeros(st.Nc))
+        n0 = dg.kernel_times().get("happly", (0, 0))[1]
+        r = dg.h_solve(g("grav"), g("theta"), g("dt"), maxiters=maxiters, precond=1, epsilon=1e-10)
+        assert r["niters"] == 0
+        assert not np.any(dg.download("h", st.Nc))
+        assert dg.kernel_times()["happly"][1] - n0 == 1, maxiters
+    dg.close()
