@@ -779,7 +779,11 @@ int sunhip_h_solve_mixed(sunhip_grid *g, const sunhip_cg_params *prm, double gra
   if (rc) return rc;
   float *c32, *f32, *x32, *r32, *z32, *t32, *pa, *pb;
   if (!g->d_h32) {
-    if ((rc = dev_alloc(g, (void **)&g->d_h32, sizeof(float) * (size_t)g->NS * (7 + g->mf)))) return rc;
+    // zero: columns that are not computational are read as neighbours but never written
+    const int n32 = g->NS * (7 + g->mf);
+    if ((rc = dev_alloc(g, (void **)&g->d_h32, sizeof(float) * (size_t)n32))) return rc;
+    k_hfill<float><<<(n32 + 255) / 256, 256, 0, g->stream>>>(g->d_h32, n32, 0.0f);
+    HIPCHK(hipGetLastError());
   }
   c32 = g->d_h32; x32 = c32 + g->NS; r32 = x32 + g->NS; z32 = r32 + g->NS; t32 = z32 + g->NS;
   pa = t32 + g->NS; pb = pa + g->NS; f32 = pb + g->NS;

@@ -101,3 +101,32 @@ def test_already_converged(gpu_available):
         assert not np.any(dg.download("h", st.Nc))
         assert dg.kernel_times()["happly"][1] - n0 == 1, maxiters
     dg.close()
+
+
+@pytest.mark.parametrize("small", [1, 0])
+def test_mixed_form_reads_no_stale_memory(gpu_available, small):
+    """The mixed form on a grid with boundary columns next to computational
+    ones, its work arrays in memory that held NaN: as on fresh memory."""
+    st = cases.tiny(4, nx=17, ny=11, Nkmax=12, open_marks=cases.open_ends())
+    st.set("D", cases.depth_integrated_D(st))
+    g = st.get_prop
+    st.set_prop(hprecond=1, epsilon=1e-12, maxiters=3000)
+    a = st.clone()
+    _impls.oracle().cgsolve(a)
+    for again in range(4):
+        dirty = [device.DeviceGrid(st) for _ in range(4)]
+        for dg in dirty:  # fields of many sizes, freed with NaN in them
+            for i in range(24):
+                dg.upload("q%d" % i, np.full(len(st.get("dzz")), np.nan))
+                dg.upload("up_%d" % i, np.full(len(st.get("u")), np.nan))
+                dg.upload("htmp%d" % (2 + i % 2), np.full(st.Nc, np.nan))
+            dg.close()
+        dg = device.DeviceGrid(st)
+        dg.tune("small", small)
+        for f in ("D", "htmp", "h"):
+            dg.upload(f, st.get(f))
+        r = dg.h_solve_mixed(g("grav"), g("theta"), g("dt"), epsilon=1e-10, precond=1)
+        h = dg.download("h", st.Nc)
+        dg.close()
+        assert r["converged"]
+        assert np.linalg.norm(h - a.get("h")) <= 1e-8 * np.linalg.norm(a.get("h"))
