@@ -202,7 +202,8 @@ int sunhip_q_coefficients(sunhip_grid *g);
  * batch call 0 for all members if it is 0 for one).  Only "tiles", "reduce",
  * "rzid", "band", "order" and "h_blocks", and "small" in the free-surface
  * solve, change the rounding of a dot product; every other knob gives
- * bit-identical results.  The pressure iteration of small grids takes every
+ * bit-identical results.  The pressure iteration of small grids (by tiles and
+ * bytes, at most 1024 tiles of 64 columns) takes every
  * operator and preconditioner knob ("unroll", "prec_unroll", "reduce",
  * "tiles", "ntstore", "rzid", "minwaves", "blocklds", "band", "prec_head",
  * "order", "xchg") at its default: setting one of them selects the kernels of

@@ -1004,7 +1004,7 @@ int sunhip_batch_begin_q_mixed(sunhip_batch *b, sunhip_grid *g, const sunhip_cg_
   Task t{};
   t.g = g; t.kind = T_QMIX; t.tag = tag;
   if ((t.stage = take_stage(b)) < 0) return -3;
-  if ((rc = q_mixed_prepare(g, prm, &t.q32, &t.R, q_seg_fits(g)))) return rc;
+  if ((rc = q_mixed_prepare(g, prm, &t.q32, &t.R, q_seg_fits(g, sizeof(float))))) return rc;
   t.mstate = M_RESID;
   t.prm = *prm;
   t.inner_tol = inner_tol;

@@ -715,7 +715,7 @@ int cg_iteration(sunhip_grid *g, const sunhip_cg_params *prm, QSolver<T> &S, int
 template <typename T>
 int cg_loop(sunhip_grid *g, const sunhip_cg_params *prm, QSolver<T> &S, int pk_apply, int pk_prec,
             bool finish = true) {
-  if (q_seg_ok(g, prm)) return q_seg_loop<T>(g, prm, S, pk_apply, pk_prec, finish);
+  if (q_seg_ok(g, prm, sizeof(T))) return q_seg_loop<T>(g, prm, S, pk_apply, pk_prec, finish);
   int rc;
   int every = prm->check_every > 0 ? prm->check_every : (g->NT > (1 << 22) ? 4 : 8);
   if (every & 1) every++;
@@ -914,7 +914,7 @@ int upload_scal(sunhip_grid *g, CGScal *d, const sunhip_cg_params *prm, CGScal *
 int q_begin64(sunhip_grid *g, const sunhip_cg_params *prm, QSolver<double> *S, CGScal *stage, CGScal *sc) {
   HIPCHK(hipSetDevice(g->device));
   F64 B;
-  const bool seg = prm->precond == 2 && q_seg_fits(g);  // the same values in three shorter launches
+  const bool seg = prm->precond == 2 && q_seg_fits(g, sizeof(double));  // the same values in three shorter launches
   int rc = q_setup(g, prm, B, *S, stage, sc, seg);
   return rc || !seg ? rc : q_seg_settle(g, S->sc);
 }
@@ -1033,7 +1033,7 @@ int sunhip_q_solve(sunhip_grid *g, const sunhip_cg_params *prm, sunhip_cg_stats 
   int rc;
   HIPCHK(hipEventRecord(g->ev0, g->stream));
   read_tuning(g);
-  const bool seg = q_seg_ok(g, prm);
+  const bool seg = q_seg_ok(g, prm, sizeof(double));
   if ((rc = q_setup(g, prm, B, S, nullptr, nullptr, seg))) return rc;
   HIPCHK(hipEventRecord(g->ev1, g->stream));
   if ((rc = cg_loop<double>(g, prm, S, PK_QAPPLY, PK_QPREC))) return rc;
@@ -1051,7 +1051,7 @@ int sunhip_q_solve_fixed(sunhip_grid *g, const sunhip_cg_params *prm, int n, sun
   int rc;
   HIPCHK(hipEventRecord(g->ev0, g->stream));
   read_tuning(g);
-  const bool seg = q_seg_ok(g, &p);
+  const bool seg = q_seg_ok(g, &p, sizeof(double));
   if ((rc = q_setup(g, &p, B, S, nullptr, nullptr, seg))) return rc;
   HIPCHK(hipEventRecord(g->ev1, g->stream));
   if ((rc = cg_loop<double>(g, &p, S, PK_QAPPLY, PK_QPREC))) return rc;
@@ -1071,7 +1071,7 @@ int sunhip_q_solve_mixed(sunhip_grid *g, const sunhip_cg_params *prm, double inn
   QSolver<float> S;
   QVec<double, float> R;
   read_tuning(g);
-  const bool seg = q_seg_ok(g, prm);
+  const bool seg = q_seg_ok(g, prm, sizeof(float));
   int rc = q_mixed_prepare(g, prm, &S, &R, seg);
   if (rc) return rc;
   CGScal *so = g->d_mo;

@@ -515,16 +515,18 @@ int seg_per_wave(const sunhip_grid *g, int most) {
 
 namespace sunhip {
 
-bool q_seg_ok(const sunhip_grid *g, const sunhip_cg_params *prm) {
+bool q_seg_ok(const sunhip_grid *g, const sunhip_cg_params *prm, size_t value_bytes) {
   // every knob of the one-lane-per-column kernels at its default
   const bool plain = g->tune_xchg < 0 && g->tune_tiles == 4 && !g->tune_blk && !g->tune_band && !g->tune_minw &&
                      g->tune_unroll == 4 && g->tune_nts && g->tune_rzid && g->tune_phead < 0 && g->tune_punroll == 8 &&
                      g->tune_reduce == 1;
-  return plain && prm->precond == 2 && q_seg_fits(g);
+  return plain && prm->precond == 2 && q_seg_fits(g, value_bytes);
 }
 
-bool q_seg_fits(const sunhip_grid *g) {
-  return g->tune_small && g->tune_order && g->Nt <= SUNHIP_QSEG_TILES && seg_count(g) <= 16;
+bool q_seg_fits(const sunhip_grid *g, size_t value_bytes) {
+  const bool size = g->Nt <= SUNHIP_QSEG_FULL ||
+                    (g->Nt <= SUNHIP_QSEG_TILES && (size_t)g->Nflat * value_bytes <= SUNHIP_QSEG_BYTES);
+  return g->tune_small && g->tune_order && size && seg_count(g) <= 16;
 }
 
 int q_seg_settle(sunhip_grid *g, CGScal *sc) {

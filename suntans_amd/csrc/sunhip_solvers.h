@@ -42,16 +42,27 @@ int set_zdz(sunhip_grid *g, const double *dz);
 int q_windows(sunhip_grid *g, const double *coef, const double *dzf, ZReg *Z);
 
 // The iteration of small and middle grids (sunhip_qseg.hip): one block per
-// tile.  At most SUNHIP_QSEG_TILES tiles, the defaults of the other kernels'
-// knobs, and qprecond=2.  Per iteration, these kernels against the
-// one-lane-per-column ones and their finishers: 32 tiles of 50 levels 27 / 69
-// us, 220 tiles of hexagons 33 / 87, 381 tiles 38 / 71, 817 tiles of 61 levels
-// 69 / 106, 790 tiles of 80 levels 87 / 117; at 1570 tiles of 80 levels 190 /
-// 135, every CU then having waves enough either way.
+// tile, with the defaults of the other kernels' knobs and qprecond=2.  It
+// takes grids of at most SUNHIP_QSEG_FULL tiles, which the chip holds at once
+// (two blocks per CU), and up to SUNHIP_QSEG_TILES while a field of the
+// computational values is at most SUNHIP_QSEG_BYTES: a segment's stores and
+// its reads of the levels above and below it miss the caches beyond that,
+// where the whole-column kernels read each value once.  Per iteration,
+// these kernels against those and their finishers, bathymetry of smooth bumps (0.55
+// of the levels filled) or flat (all filled):
+//   FP64  255 tiles of 40 levels 27 / 57 us, 508 of 70 52 / 84, 768 of 70 75 / 83,
+//         254 of hexagons of 40 32 / 74; flat: 508 of 100 110 / 115, 508 of 128
+//         143 / 158, 768 of 40 (15.8 MB) 64 / 66; but 768 of 70 (27 MB) 115 / 85,
+//         996 of 40 (20 MB) 75 / 69, 996 of 100 (51 MB) 229 / 174
+//   FP32  508 of 70 40 / 83; flat: 996 of 40 (10 MB) 54 / 62, 996 of 70 (18 MB)
+//         82 / 82, 996 of 100 (25 MB) 121 / 108
+#define SUNHIP_QSEG_FULL 512
 #define SUNHIP_QSEG_TILES 1024
-bool q_seg_ok(const sunhip_grid *g, const sunhip_cg_params *prm);
-// Whether the grid's size and dispatch order allow these kernels at all.
-bool q_seg_fits(const sunhip_grid *g);
+#define SUNHIP_QSEG_BYTES (16 << 20)
+bool q_seg_ok(const sunhip_grid *g, const sunhip_cg_params *prm, size_t value_bytes);
+// Whether the grid's size and dispatch order allow these kernels at all, for
+// values of value_bytes each.
+bool q_seg_fits(const sunhip_grid *g, size_t value_bytes);
 // The scalars at sc after their pending first step (q_seg_start), in place.
 int q_seg_settle(sunhip_grid *g, CGScal *sc);
 // Coefficients, inverse pivots and l (QSolver::ql) from dzz, or the last two

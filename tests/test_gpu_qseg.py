@@ -48,6 +48,16 @@ def test_sizes(gpu_available, nx, ny, levels):
     same(st, mixed=True)
 
 
+@pytest.mark.parametrize("nx,ny,levels", [(128, 128, 70), (145, 142, 100), (181, 181, 100), (181, 181, 128)],
+                         ids=["512 tiles", "644 tiles", "1024 tiles", "1024 deep"])
+def test_around_the_size_limits(gpu_available, nx, ny, levels):
+    """512 tiles and up to 1024, values of 10 to 34 MB in FP64 and half of
+    that in FP32: both sides of the lines to the whole-column kernels."""
+    st = cases.tiny(levels, nx=nx, ny=ny, Nkmax=levels)
+    same(st, fixed=3)
+    same(st, mixed=True)
+
+
 @pytest.mark.parametrize("fixed", [1, 2, 3])
 def test_fixed_iterations(gpu_available, fixed):
     same(cases.lock_exchange(seed=3), fixed=fixed)
