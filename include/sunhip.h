@@ -184,8 +184,8 @@ int sunhip_q_coefficients(sunhip_grid *g);
  * inside each wave through LDS, gathering only cross-tile neighbours from
  * memory: 0 off, 1 on, 2 on with a register budget of 4 waves per SIMD, 3 on
  * with 2 levels per load group, 4-6 the pipelined form; -1, the default: 0
- * below 1536 tiles of cells of at most 4 faces, else 2 for triangles and 1
- * for cells of more faces), "tvd_group" (levels per load group of the
+ * below 1536 tiles of cells of at most 4 faces and below 1024 of more, else 2
+ * for triangles and 1 for cells of more faces), "tvd_group" (levels per load group of the
  * scalar step's column update: 1, 2 (the default) or 4), "prec_lds" (levels
  * below the preconditioner's register head of 16 or 24 that keep their
  * Thomas rows in LDS between the sweeps: 0 or 12, the default), "tvd_head" (Thomas

@@ -517,11 +517,13 @@ int launch_apply(sunhip_grid *g, CGScal *sc, const QVec<T, TO> &V, const Red &R,
     // The exchange kernel, unless another launch shape was asked for.  With
     // few tiles the plain kernel at 2 levels per group has more waves in
     // flight: 790 tiles of triangles 50 us against 58, 1570 tiles 83
-    // against 80, 3900 tiles 239 against 204; with 6 or 8 faces the exchange
-    // saves most gathers at any size (1090 tiles of hexagons 114 against 86).
-    // Its register budget of 4 waves per SIMD spills from 4 faces up (780
-    // tiles of quadrilaterals 93 us against 54 without the budget).
-    const bool few = g->Nt < 1536 && g->mf <= 4;
+    // against 80, 3900 tiles 239 against 204.  With 6 or 8 faces the exchange
+    // saves more gathers and pays earlier: up to 8 faces, 320 tiles of 40
+    // levels 54 us plain against 64, 640 of 100 levels 114 / 147, 874 of 100
+    // 161 / 167, 1246 of 40 99 / 83; hexagons, 512 of 40 levels 47 / 61, 1090
+    // 114 / 86.  Its register budget of 4 waves per SIMD spills from 4 faces up
+    // (780 tiles of quadrilaterals 93 us against 54 without the budget).
+    const bool few = g->Nt < (g->mf <= 4 ? 1536 : 1024);
     const int xmode = g->tune_xchg >= 0 ? g->tune_xchg : (few ? 0 : g->mf <= 3 ? 2 : 1);
     if (zr && xmode >= 4 && g->max_pairs <= SUNHIP_XPAIRS && g->tune_unroll == 4) {
       // the pipelined exchange kernel: 4 two-level groups (xchg 4), 4 four-level
