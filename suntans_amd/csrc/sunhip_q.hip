@@ -491,7 +491,12 @@ template <int MODE, typename T, typename TO>
 int launch_apply(sunhip_grid *g, CGScal *sc, const QVec<T, TO> &V, const Red &R, int pk = -1) {
   // launch-shape variants (tiles per block, streaming stores) exist for the
   // fused iteration kernel on triangles at the default unroll
-  // (with no other shape asked for, small launches take the plain kernel below)
+  // (with no other shape asked for, launches without the exchange take the
+  // plain kernel below: few tiles, and at any size grids with a tile of more
+  // than SUNHIP_XPAIRS cross-tile faces.  It runs 2 levels per group with
+  // cached stores, whatever the size: 1600 tiles of 40 levels 70 us against
+  // 125 at 4 levels with streamed stores, 3900 of 100 622 / 809, 15600 of 100
+  // 2420 / 3131; in FP32 49 / 85, 400 / 589, 1582 / 2331)
   const bool dflt = g->tune_unroll == 4 && g->tune_xchg < 0 && g->tune_tiles == 4 && !g->tune_blk && !g->tune_band &&
                     !g->tune_minw && g->tune_nts;
   const bool variants = MODE == QM_FUSED && g->mf <= 3 && g->tune_unroll == 4 && !dflt;

@@ -70,6 +70,28 @@ def test_default_kernels_above_1024_tiles(gpu_available, kw):
     assert np.array_equal(out[0][1], out[1][1]) and np.array_equal(out[0][3], out[1][3])
 
 
+def test_plain_operator_on_scattered_tiles(gpu_available, monkeypatch):
+    """A grid of over 1536 tiles in which one tile gathers cells from all over
+    (more cross-tile faces than the exchange holds) runs the plain operator
+    by default: the same bits as at one level per group."""
+    st = cases.tiny(9, nx=230, ny=220, Nkmax=7)
+    xv, yv = st.get("xv").copy(), st.get("yv").copy()
+    i = np.random.default_rng(1).permutation(st.Nc)[:64]
+    xv[i], yv[i] = xv[i[0]], yv[i[0]]
+    top = device.topology
+    monkeypatch.setattr(device, "topology", lambda s: top(s, {"xv": xv, "yv": yv}))
+    out = []
+    for tuning in ((), (("xchg", 0), ("unroll", 1))):
+        dg = device.DeviceGrid(st)
+        device.member_upload(dg, st)
+        for k, v in tuning:
+            dg.tune(k, v)
+        n = dg.q_solve(epsilon=1e-10)["niters"]
+        out.append((n, dg.download("q", dg.sizes()["Nflat"])))
+        dg.close()
+    assert out[0][0] == out[1][0] and np.array_equal(out[0][1], out[1][1])
+
+
 @pytest.mark.parametrize("levels", [23, 24, 25, 33, 50])
 def test_entry_above_1024_tiles(gpu_available, levels):
     """The Preconditioner entry with its 24-row register head (1024 tiles and
