@@ -440,11 +440,28 @@ int launch_prec(sunhip_grid *g, CGScal *sc, const T *coef, const T *z, T *r, T *
   // 390 and 467 us in FP64 (40: 2 waves per SIMD, 48 spills) and 231, 212,
   // 219 and 207 us in FP32; without the LDS stage 32 levels take 485 and
   // 248 us.  Few tiles (below 1024) take the plain sweep.
-  const bool fp32 = std::is_same<T, float>::value;
   const bool nt = g->NT * (int64_t)sizeof(T) >= SUNHIP_STREAM_BYTES;
-  const int head = g->tune_phead >= 0 ? g->tune_phead : (g->Nt >= 1024 ? 40 : 0);
+  const int head = g->tune_phead >= 0 ? g->tune_phead : (g->Nt >= 1024 ? QHead<T>::regs : 0);
+  // the default head; cached stores while the vectors stay in the memory-side
+  // cache (see launch_apply)
+  auto head_lds = [&](auto ntc) {
+    constexpr bool NT = decltype(ntc)::value;
+    if (zr)
+      k_qprec<UPDATE, 4, T, true, QHead<T>::regs, true, QHead<T>::lds, NT>
+          <<<nb, 256, 0, g->stream>>>(G, coef, z, r, out, bq, sc, R, ZZ);
+    else
+      k_qprec<UPDATE, 4, T, true, QHead<T>::regs, false, QHead<T>::lds, NT>
+          <<<nb, 256, 0, g->stream>>>(G, coef, z, r, out, bq, sc, R, ZZ);
+  };
+  const bool dhead = head == QHead<T>::regs && rzid;
   if constexpr (!UPDATE) {
-    PREC(4, 0);  // once per solve; every variant gives the same bits
+    // once per solve; every variant gives the same bits.  A whole solve of one
+    // iteration with the head and with every row through memory: 1993 tiles of
+    // 40 levels 485 / 566 us, 7986 of 100 4372 / 5162, 3993 of hexagons of 100
+    // 2954 / 3351
+    if (dhead && nt) head_lds(std::true_type{});
+    else if (dhead) head_lds(std::false_type{});
+    else PREC(4, 0);
   } else if (head == 0) {
     switch (g->tune_punroll) {
       case 1: PREC(1, 0); break;
@@ -465,16 +482,9 @@ int launch_prec(sunhip_grid *g, CGScal *sc, const T *coef, const T *z, T *r, T *
         break;
       case 32: PREC(4, 32); break;
       default:
-        if (rzid && !nt) {  // the vectors stay in the memory-side cache (see launch_apply)
-          if (zr)
-            k_qprec<UPDATE, 4, T, true, QHead<T>::regs, true, QHead<T>::lds, false>
-                <<<nb, 256, 0, g->stream>>>(G, coef, z, r, out, bq, sc, R, ZZ);
-          else
-            k_qprec<UPDATE, 4, T, true, QHead<T>::regs, false, QHead<T>::lds, false>
-                <<<nb, 256, 0, g->stream>>>(G, coef, z, r, out, bq, sc, R, ZZ);
-        } else {
-          PREC3(4, QHead<T>::regs, QHead<T>::lds);
-        }
+        if (dhead && nt) head_lds(std::true_type{});
+        else if (dhead) head_lds(std::false_type{});
+        else PREC3(4, QHead<T>::regs, QHead<T>::lds);  // rz from the backward sweep
         break;
     }
   }
