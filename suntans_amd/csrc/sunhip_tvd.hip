@@ -44,17 +44,28 @@ __global__ __launch_bounds__(256) void k_tvd_faces(Geo G, TvdArgs A, Bands B) {
 // The column update by segments (update_column_seg), one block per tile.  A
 // lane that walks a whole column waits out each level's loads and nine
 // divisions in turn (50 levels: 97 us on any grid); with a wave per 8 levels
-// only the elimination is serial.  The rows take 214 VGPRs and up, one block
-// per CU, so it pays while there are few blocks per CU: 129 tiles of 37 levels
-// 78 -> 34 us, 500 of 50 103 -> 71, 820 of 61 levels 131 -> 132; with 16 levels
-// per wave (more than 64 levels) 75 tiles of 100 levels 193 -> 76 us, 240 of
-// 90 176 -> 75, but spills cost more than it gives from 6 faces (280 tiles
-// of 67 levels 141 -> 155).  First-order upwind (pre false) gathers its fluxes
-// here and spills from 6 faces too; 129 tiles of quadrilaterals 65 -> 40 us.
+// only the elimination is serial.  The rows take 214 VGPRs and up, 8 waves per
+// CU, so it pays while there are few blocks per CU and a column has more than
+// one segment: 129 tiles of 37 levels 78 -> 34 us, 500 of 50 103 -> 71, 500 of
+// 64 (smooth or random depths, any faces) half the whole columns' time; 512 of 5
+// levels, one wave either way, 21.2 -> 22.4.  Past two blocks per CU only
+// blocks that fill a CU's 8 waves still do: 740 tiles of 12, 30, 52 and 64
+// levels 33 -> 31, 67 -> 60, 109 -> 106 and 138 -> 115, but of 20, 40 and 44
+// levels 48 -> 54, 86 -> 92 and 93 -> 96 (hexagons of 20 and 44 52 -> 62 and
+// 102 -> 108).  With 16 levels per wave (more than 64 levels) 75 tiles of 100
+// levels 193 -> 76 us, 240 of 90 176 -> 75, but spills cost more than it gives
+// from 6 faces (280 tiles of 67 levels 141 -> 155).
+// First-order upwind (pre false) gathers its fluxes here, and spills more the
+// more faces: triangles of up to 64 levels 500 tiles of 40 0.94 of the whole
+// columns' time, 640 1.31; quadrilaterals 239 tiles of 40 70 -> 44, 300 of 40
+// and 90 levels 71 -> 72 and 152 -> 194.
 template <int NF>
 static bool tvd_seg(const sunhip_grid *g, bool pre) {
-  if (!g->tune_small || g->tune_tvdgrp != 2 || g->tune_tvdhead != 8 || (!pre && NF > 4)) return false;
-  return g->maxdepth <= 8 * SUNHIP_SEG ? g->Nt <= 768 : NF <= 4 && g->maxdepth <= 16 * SUNHIP_SEG && g->Nt <= 512;
+  if (!g->tune_small || g->tune_tvdgrp != 2 || g->tune_tvdhead != 8) return false;
+  const int ns = (g->maxdepth + SUNHIP_SEG - 1) / SUNHIP_SEG;
+  if (ns < 2 || ns > (NF <= 4 ? 16 : 8) || (!pre && NF > 4)) return false;
+  if (!pre) return g->Nt <= (NF == 3 && ns <= 8 ? 512 : 256);
+  return g->Nt <= (ns <= 8 && 8 / ns * ns >= 7 ? 768 : 512);
 }
 template <int NF, bool PRE, int SPW>
 __global__ __launch_bounds__(512, 2) void k_update_column_seg(Geo G, ColArgs A) {
