@@ -129,7 +129,11 @@ int face_scalars_launch(sunhip_grid *g, const TvdArgs &A) {
   int ps = prof_begin(g, PK_TSUMS);
   with_nf(g->mf, [&](auto nf) {
     constexpr int NF = decltype(nf)::value;
-    const Bands B = level_bands(g, g->Nt);
+    Bands B = level_bands(g, g->Nt);
+    // two bands of a shallow column of many faces cost more set-up than they
+    // share: hexagons of 12 levels 512 tiles 0.69 of the whole columns' time,
+    // 699 1.10, 2998 1.12; of 100 levels 0.64, 0.85, 0.95
+    if (NF >= 6 && g->Nt > 512 && g->maxdepth <= 16) B.nb = 1;
     const unsigned nb = (unsigned)((g->Nt + 3) / 4), nbb = (unsigned)(((int64_t)g->Nt * B.nb + 3) / 4);
     if (g->tune_sumsgrp == 4 && B.nb > 1) k_tvd_sums<NF, 4, true><<<nbb, 256, 0, g->stream>>>(G, A, B);
     else if (g->tune_sumsgrp == 4) k_tvd_sums<NF, 4><<<nb, 256, 0, g->stream>>>(G, A);
