@@ -90,34 +90,38 @@ sunhip::Geo sunhip_grid::geo() const {
 }
 
 // ---------------------------------------------------------------------------
-// staging kernels: a block transposes SBAND levels of one tile through LDS.
+// staging kernels: a block transposes SB levels of one tile through LDS.
 // A column's values are contiguous in the flat array and 64 apart in the
 // tile, so one thread per column touched a cache line per value on the flat
-// side; here a half wave moves 32 values of a column at a time, and a column's
+// side; here SB lanes move SB values of a column at a time, and a column's
 // levels are not walked in turn.  Over the cell and edge fields of 250k
 // columns of 100 levels: to the flat order 285 -> 126 us, to the tiles 155 ->
-// 113; of 2000 columns of 50 levels 7 us each.
-constexpr int SBAND = 32;
+// 113; of 2000 columns of 50 levels 7 us each.  Shallow grids take SB = 8 or
+// 16, whose lanes all have levels: an upload of 5000 tiles of 5 levels 382 us at
+// SB = 32 and 367 at 8 (one thread per column 364), of 15000 of 12 levels 2572
+// and 2413 (2428).
 
 // The tile and first level of a block: nband blocks per tile.
+template <int SB>
 __device__ __forceinline__ int stage_tile(int nband, int &k0) {
   const int t = blockIdx.x / nband;
-  k0 = (blockIdx.x - t * nband) * SBAND;
+  k0 = (blockIdx.x - t * nband) * SB;
   return t;
 }
 
+template <int SB>
 __global__ __launch_bounds__(256) void k_scatter_cols(const double *__restrict__ flat, double *__restrict__ dst,
                                                       const int64_t *__restrict__ fstart, const int *__restrict__ ncol,
                                                       int extra, const int *__restrict__ toff,
                                                       const int *__restrict__ tdep, int nband) {
-  __shared__ double sh[SBAND][SUNHIP_TILE + 1];
+  __shared__ double sh[SB][SUNHIP_TILE + 1];
   int k0;
-  const int t = stage_tile(nband, k0), d = tdep[t];
+  const int t = stage_tile<SB>(nband, k0), d = tdep[t];
   if (k0 >= d) return;
-  const int kk = threadIdx.x & (SBAND - 1);
+  const int kk = threadIdx.x % SB;
 #pragma unroll
-  for (int j = 0; j < SUNHIP_TILE; j += 256 / SBAND) {
-    const int c = j + (threadIdx.x >> 5), s = t * SUNHIP_TILE + c;
+  for (int j = 0; j < SUNHIP_TILE; j += 256 / SB) {
+    const int c = j + threadIdx.x / SB, s = t * SUNHIP_TILE + c;
     const int64_t f0 = fstart[s];
     const int n = f0 < 0 ? 0 : ncol[s] + extra;
     sh[kk][c] = k0 + kk < n ? flat[f0 + k0 + kk] : 0.0;
@@ -125,34 +129,43 @@ __global__ __launch_bounds__(256) void k_scatter_cols(const double *__restrict__
   __syncthreads();
   const int l = threadIdx.x & 63;
 #pragma unroll
-  for (int j = 0; j < SBAND; j += 4) {
+  for (int j = 0; j < SB; j += 4) {
     const int r = j + (threadIdx.x >> 6);
     if (k0 + r < d) dst[toff[t] + (int64_t)(k0 + r) * SUNHIP_TILE + l] = sh[r][l];
   }
 }
 
+template <int SB>
 __global__ __launch_bounds__(256) void k_gather_cols(double *__restrict__ flat, const double *__restrict__ src,
                                                      const int64_t *__restrict__ fstart, const int *__restrict__ ncol,
                                                      int extra, const int *__restrict__ toff,
                                                      const int *__restrict__ tdep, int nband) {
-  __shared__ double sh[SBAND][SUNHIP_TILE + 1];
+  __shared__ double sh[SB][SUNHIP_TILE + 1];
   int k0;
-  const int t = stage_tile(nband, k0), d = tdep[t];
+  const int t = stage_tile<SB>(nband, k0), d = tdep[t];
   if (k0 >= d) return;
   const int l = threadIdx.x & 63;
 #pragma unroll
-  for (int j = 0; j < SBAND; j += 4) {
+  for (int j = 0; j < SB; j += 4) {
     const int r = j + (threadIdx.x >> 6);
     if (k0 + r < d) sh[r][l] = src[toff[t] + (int64_t)(k0 + r) * SUNHIP_TILE + l];
   }
   __syncthreads();
-  const int kk = threadIdx.x & (SBAND - 1);
+  const int kk = threadIdx.x % SB;
 #pragma unroll
-  for (int j = 0; j < SUNHIP_TILE; j += 256 / SBAND) {
-    const int c = j + (threadIdx.x >> 5), s = t * SUNHIP_TILE + c;
+  for (int j = 0; j < SUNHIP_TILE; j += 256 / SB) {
+    const int c = j + threadIdx.x / SB, s = t * SUNHIP_TILE + c;
     const int64_t f0 = fstart[s];
     if (f0 >= 0 && k0 + kk < ncol[s] + extra) flat[f0 + k0 + kk] = sh[kk][c];
   }
+}
+
+// fn(std::integral_constant<int, SB>) for tiles of depth levels.
+template <typename F>
+static void with_stage(int depth, F &&fn) {
+  if (depth <= 8) fn(std::integral_constant<int, 8>{});
+  else if (depth <= 16) fn(std::integral_constant<int, 16>{});
+  else fn(std::integral_constant<int, 32>{});
 }
 
 __global__ void k_scatter_2d(const double *__restrict__ flat, double *__restrict__ dst,
@@ -803,14 +816,22 @@ static int pinned_slot(const sunhip_grid *g, const double *flat, size_t n) {
 }  // extern "C"
 
 static void scatter_field(sunhip_grid *g, const Field *f, const double *st) {
-  const int nc = (g->maxdepth + 1 + SBAND - 1) / SBAND, ne = (g->maxedepth + SBAND - 1) / SBAND;
   switch (f->kind) {
     case CELL: case CELLW:
-      k_scatter_cols<<<g->Nt * nc, 256, 0, g->stream>>>(st, f->d, f->kind == CELL ? g->d_cstart : g->d_cstartw, g->d_nk,
-                                                        f->kind == CELLW, g->d_toff, g->d_tdep, nc);
+      with_stage(g->maxdepth + 1, [&](auto sb) {
+        constexpr int SB = decltype(sb)::value;
+        const int nb = (g->maxdepth + SB) / SB;
+        k_scatter_cols<SB><<<g->Nt * nb, 256, 0, g->stream>>>(st, f->d, f->kind == CELL ? g->d_cstart : g->d_cstartw,
+                                                              g->d_nk, f->kind == CELLW, g->d_toff, g->d_tdep, nb);
+      });
       break;
     case EDGE:
-      k_scatter_cols<<<g->Net * ne, 256, 0, g->stream>>>(st, f->d, g->d_estart, g->d_e_nkc, 0, g->d_eoff, g->d_edep, ne);
+      with_stage(g->maxedepth, [&](auto sb) {
+        constexpr int SB = decltype(sb)::value;
+        const int nb = (g->maxedepth + SB - 1) / SB;
+        k_scatter_cols<SB><<<g->Net * nb, 256, 0, g->stream>>>(st, f->d, g->d_estart, g->d_e_nkc, 0, g->d_eoff,
+                                                               g->d_edep, nb);
+      });
       break;
     case CELL2:
       k_scatter_2d<<<(g->Nc + 255) / 256, 256, 0, g->stream>>>(st, f->d, g->d_cellslot, g->Nc);
@@ -822,14 +843,22 @@ static void scatter_field(sunhip_grid *g, const Field *f, const double *st) {
 }
 
 static void gather_field(sunhip_grid *g, const Field *f, double *st) {
-  const int nc = (g->maxdepth + 1 + SBAND - 1) / SBAND, ne = (g->maxedepth + SBAND - 1) / SBAND;
   switch (f->kind) {
     case CELL: case CELLW:
-      k_gather_cols<<<g->Nt * nc, 256, 0, g->stream>>>(st, f->d, f->kind == CELL ? g->d_cstart : g->d_cstartw, g->d_nk,
-                                                       f->kind == CELLW, g->d_toff, g->d_tdep, nc);
+      with_stage(g->maxdepth + 1, [&](auto sb) {
+        constexpr int SB = decltype(sb)::value;
+        const int nb = (g->maxdepth + SB) / SB;
+        k_gather_cols<SB><<<g->Nt * nb, 256, 0, g->stream>>>(st, f->d, f->kind == CELL ? g->d_cstart : g->d_cstartw,
+                                                             g->d_nk, f->kind == CELLW, g->d_toff, g->d_tdep, nb);
+      });
       break;
     case EDGE:
-      k_gather_cols<<<g->Net * ne, 256, 0, g->stream>>>(st, f->d, g->d_estart, g->d_e_nkc, 0, g->d_eoff, g->d_edep, ne);
+      with_stage(g->maxedepth, [&](auto sb) {
+        constexpr int SB = decltype(sb)::value;
+        const int nb = (g->maxedepth + SB - 1) / SB;
+        k_gather_cols<SB><<<g->Net * nb, 256, 0, g->stream>>>(st, f->d, g->d_estart, g->d_e_nkc, 0, g->d_eoff,
+                                                              g->d_edep, nb);
+      });
       break;
     case CELL2:
       k_gather_2d<<<(g->Nc + 255) / 256, 256, 0, g->stream>>>(st, f->d, g->d_cellslot, g->Nc);
