@@ -85,7 +85,6 @@ sunhip::Geo sunhip_grid::geo() const {
   G.df = d_df; G.dg = d_dg;
   G.xcode = d_xcode; G.pair = d_pair; G.npair = d_npair;
   G.b4perm = tune_order ? d_b4perm : nullptr;
-  G.b4inv = d_b4inv;
   return G;
 }
 
@@ -593,14 +592,13 @@ int sunhip_grid_create(sunhip_grid **out, const sunhip_topology *T, int device) 
                        [&](int a, int b) { return gdep[a] > gdep[b]; });
       start += len;
     }
-    rc |= upload_vec(g, &g->d_b4perm, perm);
     // block v works on group perm[u], u the v-th block's place in its XCD's run
-    std::vector<int> inv(nb4);
+    perm.resize(2 * (size_t)nb4);
     for (int v = 0; v < nb4; v++) {
       const int x = v & 7, u = x * q + std::min(x, r8) + (v >> 3);
-      inv[perm[u]] = v;
+      perm[nb4 + perm[u]] = v;
     }
-    rc |= upload_vec(g, &g->d_b4inv, inv);
+    rc |= upload_vec(g, &g->d_b4perm, perm);
   }
   rc |= upload_vec(g, &g->d_e_nke, ezeros);
   rc |= upload_vec(g, &g->d_e_etop, ezeros);
@@ -645,7 +643,7 @@ int sunhip_grid_destroy(sunhip_grid *g) {
                   g->d_e_etop, g->d_e_mark, g->d_e_comp, g->d_cstart, g->d_cstartw, g->d_estart,
                   g->d_cellslot, g->d_edgeslot, g->d_stage[0], g->d_stage[1], g->d_stage[2], g->d_stage[3], g->d_part, g->d_count, g->d_qs, g->d_hs,
                   g->d_class_tiles, g->d_ms, g->d_mo, g->d_D32, g->d_h32, g->d_uerr, g->d_dz, g->d_e_etopold,
-                  g->d_ford, g->d_zdzt, g->d_cwin, g->d_fwin, g->d_cex, g->d_fex, g->d_tflag, g->d_b4perm, g->d_b4inv};
+                  g->d_ford, g->d_zdzt, g->d_cwin, g->d_fwin, g->d_cex, g->d_fex, g->d_tflag, g->d_b4perm};
   for (void *p : ptrs) if (p) hipFree(p);
   for (int i = 0; i < SUNHIP_PIN_SLOTS; i++) {
     if (g->h_pin[i]) hipHostFree(g->h_pin[i]);

@@ -101,10 +101,9 @@ struct Geo {
   // dispatch order of the 4-tile blocks of the column kernels (b4perm[v] =
   // the block group of virtual block v): within each XCD's run of groups the
   // deepest go first, so the launch does not end on a few deep columns;
-  // null: identity
+  // null: identity.  The inverse follows it: b4perm[groups + g] = the block
+  // whose group tile_group gives as g
   const int *b4perm;
-  // the inverse: b4inv[g] = the block whose group tile_group gives as g
-  const int *b4inv;
 };
 
 }  // namespace sunhip
@@ -132,8 +131,7 @@ struct sunhip_grid {
   int *d_nk = nullptr, *d_ctop = nullptr, *d_ctopold = nullptr, *d_comp = nullptr, *d_nf = nullptr;
   int *d_nbb = nullptr, *d_nbs = nullptr, *d_eb = nullptr, *d_es = nullptr, *d_nrm = nullptr, *d_kr = nullptr;
   int *d_xcode = nullptr, *d_pair = nullptr, *d_npair = nullptr;  // neighbour exchange (Geo)
-  int *d_b4perm = nullptr;          // depth-first dispatch order of 4-tile blocks (Geo)
-  int *d_b4inv = nullptr;           // its inverse (Geo)
+  int *d_b4perm = nullptr;          // depth-first dispatch order of 4-tile blocks and its inverse (Geo)
   int tune_order = 1;               // 1: use it
   int tune_small = 1;               // 1: small grids run kernels of their own (segments, bands, one block)
   int tune_tvdgrp = 2;              // levels per load group of the scalar column update (1, 2, 4)

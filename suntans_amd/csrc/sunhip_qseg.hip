@@ -252,7 +252,7 @@ __device__ __forceinline__ int seg_tile(const Geo &G, int b, int &pos) {
   const int nb4 = (G.Nt + 3) >> 2, q = nb4 >> 3, r = nb4 & 7, x = b & 7, i = b >> 3;
   if ((i >> 2) >= q + (x < r ? 1 : 0)) return G.Nt;
   const int g = x * q + min(x, r) + (i >> 2), t = g * 4 + (i & 3);
-  if (t < G.Nt) pos = G.b4inv[g] * 4 + (t & 3);
+  if (t < G.Nt) pos = G.b4perm[nb4 + g] * 4 + (t & 3);
   return t;
 }
 
