@@ -614,9 +614,12 @@ int sunhip_grid_create(sunhip_grid **out, const sunhip_topology *T, int device) 
   rc |= dev_alloc(g, (void **)&g->d_mo, sizeof(CGScal));
   if (rc) { sunhip_grid_destroy(g); return rc; }
   HIPCHK(hipMemset(g->d_count, 0, sizeof(unsigned) * 64));
-  HIPCHK(hipHostMalloc((void **)&g->h_sc, sizeof(CGScal), hipHostMallocDefault));
-  HIPCHK(hipHostMalloc((void **)&g->h_poll, 2 * sizeof(CGScal), hipHostMallocDefault));
-  HIPCHK(hipHostMalloc((void **)&g->h_prog, sizeof(unsigned long long), hipHostMallocDefault));
+  // the pinned scalars: the mirror, two polling slots and the progress word
+  // (on a cache line of its own) in one allocation
+  constexpr size_t prog_at = (3 * sizeof(CGScal) + 63) / 64 * 64;
+  HIPCHK(hipHostMalloc((void **)&g->h_sc, prog_at + 64, hipHostMallocDefault));
+  g->h_poll = g->h_sc + 1;
+  g->h_prog = (unsigned long long *)((char *)g->h_sc + prog_at);
   *g->h_prog = 0;
   HIPCHK(hipEventCreateWithFlags(&g->evp[0], hipEventDisableTiming));
   HIPCHK(hipEventCreateWithFlags(&g->evp[1], hipEventDisableTiming));
@@ -658,8 +661,6 @@ int sunhip_grid_destroy(sunhip_grid *g) {
   if (g->xstream) hipStreamDestroy(g->xstream);
   if (g->xdown) hipStreamDestroy(g->xdown);
   if (g->h_sc) hipHostFree(g->h_sc);
-  if (g->h_poll) hipHostFree(g->h_poll);
-  if (g->h_prog) hipHostFree(g->h_prog);
   for (hipEvent_t e : g->evp) if (e) hipEventDestroy(e);
   if (g->ev0) hipEventDestroy(g->ev0);
   if (g->ev1) hipEventDestroy(g->ev1);
