@@ -223,8 +223,8 @@ struct sunhip_grid {
   int tune_xchg = -1;    // operator kernel with the neighbour exchange inside each wave: 0 off, 1 on,
                          // 2 on with a 4-waves-per-SIMD register budget, 3 on with 2 levels per group,
                          // -1 (default) by size and face count (launch_apply)
-  int tune_phead = -1;   // top levels per column the preconditioner keeps in registers (0, 8, 16, 24, 32);
-                         // -1 (default) QHead's from 1024 tiles up, 0 below
+  int tune_phead = -1;   // top levels per column the preconditioner keeps in registers (0, 8, 16, 24, 32; 40:
+                         // QHead's); -1 (default) QHead's from 1024 tiles up, 0 below
   int tune_band = 0;     // operator kernel over level bands of this many levels (0: whole columns)
 
   // per-kernel timing (sunhip_profile): an event pair around every launch of

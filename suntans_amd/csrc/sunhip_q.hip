@@ -441,7 +441,8 @@ int launch_prec(sunhip_grid *g, CGScal *sc, const T *coef, const T *z, T *r, T *
   // 219 and 207 us in FP32; without the LDS stage 32 levels take 485 and
   // 248 us.  Few tiles (below 1024) take the plain sweep.
   const bool nt = g->NT * (int64_t)sizeof(T) >= SUNHIP_STREAM_BYTES;
-  const int head = g->tune_phead >= 0 ? g->tune_phead : (g->Nt >= 1024 ? QHead<T>::regs : 0);
+  const int head = g->tune_phead < 0 ? (g->Nt >= 1024 ? QHead<T>::regs : 0)
+                                     : (g->tune_phead == 40 ? QHead<T>::regs : g->tune_phead);
   // the default head; cached stores while the vectors stay in the memory-side
   // cache (see launch_apply)
   auto head_lds = [&](auto ntc) {
@@ -1203,8 +1204,9 @@ int sunhip_set_tuning(sunhip_grid *g, const char *key, int value) {
     g->tune_punroll = value;
   }
   else if (!strcmp(key, "prec_head")) {
-    if (value != -1 && value != 0 && value != 8 && value != 16 && value != 24 && value != 32) {
-      set_error("prec_head must be -1, 0, 8, 16, 24 or 32");
+    if (value != -1 && value != 0 && value != 8 && value != 16 && value != 24 && value != 32 &&
+        value != 40) {
+      set_error("prec_head must be -1, 0, 8, 16, 24, 32 or 40");
       return -1;
     }
     g->tune_phead = value;

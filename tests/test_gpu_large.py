@@ -3,8 +3,8 @@ bumps, up to 100 levels of 2 m, source = ComputeQSource of seeded smooth u
 and w) built at reduced planform size with the same bathymetry statistics,
 against the oracle.  The kernel variants the full size selects by default
 (the in-wave neighbour exchange of the operator, "xchg" 2, and the
-register-held top of the preconditioner, "prec_head" 24 in FP64 and 16 in
-FP32) are forced here, since the reduced grid would otherwise pick the small
+preconditioner's register head and LDS stage, "prec_head" 40, with the z-level
+windows) are forced here, since the reduced grid would otherwise pick the small
 defaults; the defaults are run too.
 
 Tolerances (FP64 pressure and free-surface solves, as the reference's CG
@@ -67,8 +67,8 @@ def _dev(st, tuning):
     return dg
 
 
-TUNINGS = [("default", {}), ("full_size_kernels", {"xchg": 2, "prec_head": 24}),
-           ("xchg3_head16", {"xchg": 3, "prec_head": 16})]
+TUNINGS = [("default", {}), ("full_size_kernels", {"xchg": 2, "prec_head": 40}),
+           ("xchg2_head24", {"xchg": 2, "prec_head": 24}), ("xchg3_head16", {"xchg": 3, "prec_head": 16})]
 
 
 def test_large_case_shape():
@@ -106,7 +106,7 @@ def test_large_q_fixed_iterations(gpu_available, n):
     a.set_prop(qprecond=2, qepsilon=0.0, qmaxiters=n)
     b = a.clone()
     o.cgsolveq(a)
-    dg = _dev(b, {"xchg": 2, "prec_head": 24})
+    dg = _dev(b, {"xchg": 2, "prec_head": 40})
     r = dg.q_solve(maxiters=n, precond=2, epsilon=0.0, fixed=n)
     q = dg.download("q", len(a.get("qc")))
     dg.close()
@@ -142,7 +142,7 @@ def _q_residual(o, st, q):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("inner_tol", [1e-4, 1e-3])
-@pytest.mark.parametrize("head", [16, -1])
+@pytest.mark.parametrize("head", [16, 40, -1])
 def test_large_q_mixed(gpu_available, inner_tol, head):
     o = _impls.oracle()
     st = large()

@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 BITWISE = [("xchg", 4), ("xchg", 5), ("xchg", 6), ("unroll", 1), ("unroll", 2), ("unroll", 8), ("prec_unroll", 1),
            ("prec_unroll", 4), ("ntstore", 0),
            ("minwaves", 3), ("minwaves", 4), ("blocklds", 1), ("prec_head", 0), ("prec_head", 8),
-           ("prec_head", 16), ("prec_head", 24), ("prec_head", 32), ("xchg", 1), ("xchg", 2), ("xchg", 3),
+           ("prec_head", 16), ("prec_head", 24), ("prec_head", 32), ("prec_head", 40), ("xchg", 1), ("xchg", 2), ("xchg", 3),
            ("zreg", 0)]
 ROUNDING = [("tiles", 8), ("tiles", 16), ("rzid", 0), ("band", 8), ("band", 16), ("band", 32), ("order", 0)]
 
@@ -41,11 +41,15 @@ def grids():
 
 @pytest.mark.parametrize("key,value", BITWISE, ids=[f"{k}={v}" for k, v in BITWISE])
 def test_variant_bitwise(gpu_available, grids, key, value):
+    """Against the kernels of large grids at their defaults (most knobs select
+    those by themselves, "zreg" does not) and against the default of these
+    grids."""
     for st in grids:
-        q0, n0 = solve(st, [])
-        q1, n1 = solve(st, [(key, value)])
-        assert n0 == n1
-        assert np.array_equal(q0, q1)
+        q1, n1 = solve(st, [("small", 0), (key, value)])
+        for base in ([("small", 0)], []):
+            q0, n0 = solve(st, base)
+            assert n0 == n1
+            assert np.array_equal(q0, q1)
 
 
 @pytest.mark.parametrize("head", [16, 24])
@@ -71,7 +75,7 @@ def test_prec_lds_bitwise(gpu_available, grids, head, rzid):
 def test_variant_rounding(gpu_available, grids, key, value):
     for st in grids:
         q0, n0 = solve(st, [])
-        q1, n1 = solve(st, [(key, value)])
+        q1, n1 = solve(st, [("small", 0), (key, value)])
         assert abs(n0 - n1) <= 1
         assert np.linalg.norm(q1 - q0) <= 1e-12 * np.linalg.norm(q0)
 
@@ -109,8 +113,10 @@ def test_zreg_bitwise_heads(gpu_available, grids, head):
 
 def scalar_step(st, group, tvd, head=0):
     """One UpdateScalars on the device with tvd_group and tvd_sums_group =
-    group and tvd_head = head; returns the new scalar and Cn."""
+    group and tvd_head = head, in the whole-column kernels that these knobs
+    shape; returns the new scalar and Cn."""
     dg = device.DeviceGrid(st)
+    dg.tune("small", 0)
     for f in ("s", "u", "utmp2", "dzf", "dzz", "dzzold", "kappa_tv", "wnew", "wtmp2"):
         dg.upload(f, st.get(f))
     dg.upload("active", st.active().astype(np.float64))
