@@ -16,7 +16,11 @@ pytestmark = pytest.mark.gpu
 SIZES = [(8, 4), (32, 16), (27, 19), (32, 32), (41, 25), (64, 32), (50, 41)]
 SHAPES = {"quad": dict(planform="quad", split_every=3, nx=40, ny=40), "hex": dict(planform="hex", nx=40, ny=25),
           "hex8": dict(planform="hex", split_every=4, maxfaces=7, nx=45, ny=40),
-          "open": dict(nx=40, ny=20, open_marks=cases.open_ends())}
+          "open": dict(nx=40, ny=20, open_marks=cases.open_ends()),
+          # just past one block: 4200 quadrilaterals, 2255 hexagons, some cells of 7 faces
+          "quad two launches": dict(planform="quad", split_every=3, nx=60, ny=60),
+          "hex two launches": dict(planform="hex", nx=55, ny=41),
+          "hex8 two launches": dict(planform="hex", split_every=4, maxfaces=7, nx=55, ny=41)}
 
 
 def check(st, precond=1):
