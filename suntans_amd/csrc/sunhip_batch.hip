@@ -224,7 +224,9 @@ __global__ void kb_gather(CGScal *const *__restrict__ src, CGScal *__restrict__ 
 // 379 -> 285, Corrector 244 -> 214, and Continuity by segments 730 -> 550.
 // Whole columns against bands and segments, calls over 12 members: 20,800
 // items source 746 / 730 us, Corrector and Continuity 1890 / 2072, scalar step
-// 2722 / 2662; 47,000 items 1517 / 1607, 3630 / 4628, 5600 / 5423.
+// 2722 / 2662; 47,000 items 1517 / 1607, 3630 / 4628, 5600 / 5423.  The line is
+// the source's and the Corrector's; the scalar passes, kept on the same one,
+// would gain 2 to 3% of a step by bands beyond it.
 static Bands batch_bands(int items, int depth, bool small) {
   if (items > 16384 || !small) return Bands{1, 0x3fffffff};
   return Bands{(depth + 1 + 31) / 32, 32};

@@ -14,10 +14,12 @@
 // solve is reproducible run to run.  Element-wise arithmetic keeps the
 // reference's operation order and is built without FMA contraction, so
 // OperatorQ and the Preconditioner entry point agree with the reference bit
-// for bit.  Inside a solve the preconditioner multiplies by inverse pivots
-// formed once, where the reference divides twice per level and application,
-// and the dot products are summed in another order.  Small and middle grids
-// run the iteration of sunhip_qseg.hip.
+// for bit.  Inside a solve the preconditioner inverts each pivot and
+// multiplies by it, one division per level and application where the
+// reference has five (the rows that go through memory read the inverse formed
+// once per solve on the way back up), and the dot products are summed in
+// another order.  Small and middle grids run the iteration of
+// sunhip_qseg.hip, which reads all its inverse pivots.
 //
 // The kernels are templated on the storage type T of vectors and
 // coefficients.  T=double is the drop-in; T=float is the inner solve of the

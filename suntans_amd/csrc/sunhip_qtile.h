@@ -1253,22 +1253,9 @@ __device__ __forceinline__ void qfinish_tile(const Geo &G, T *__restrict__ x, co
   }
 }
 
-// x64 += e32 over tile t (mixed form, FP64 accumulation).
-__device__ __forceinline__ void mix_update_tile(const Geo &G, double *__restrict__ x, const float *__restrict__ e,
-                                                int t, int l) {
-  if (t >= G.Nt) return;
-  const int s = t * 64 + l, n = G.nk[s];
-  if (n == 0 || G.comp[s] != 1) return;
-  const int64_t base = G.toff[t] + l;
-  for (int k = G.ctop[s]; k < n; k++) {
-    const int64_t idx = base + (int64_t)k * 64;
-    x[idx] = x[idx] + (double)e[idx];
-  }
-}
-
 // The inner FP32 solve's last x update (qfinish_tile, when upd) and then
-// x64 += e32 (mix_update_tile) in one pass over tile t, with the same
-// roundings as the two passes; levels [ka, kz).
+// x64 += e32 over tile t in one pass, each rounded as if they were two;
+// levels [ka, kz).
 __device__ __forceinline__ void mix_finish_tile(const Geo &G, double *__restrict__ x, const float *__restrict__ e,
                                                 const float *__restrict__ p, float nu, bool upd, int t, int l,
                                                 int ka = 0, int kz = 0x7fffffff) {

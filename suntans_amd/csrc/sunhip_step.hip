@@ -80,7 +80,6 @@ int sunhip_compute_qsource(sunhip_grid *g, double theta, double dt, const char *
   StepArgs A;
   int rc = step_args(g, theta, dt, "q", "qp", "w", src, &A);
   if (rc) return rc;
-  const Geo G = g->geo();
   const int tiles = std::max(g->Nt, g->Net), nb = (tiles + 3) / 4;
   const Bands B = level_bands(g, tiles);
   const int ps = prof_begin(g, PK_QSOURCE);
