@@ -33,7 +33,8 @@ HBM_PEAK_GBS = 8000.0  # MI355X HBM3E, vendor figure
 PMC_SUMMARY = os.path.join(ROOT, "profiles", "pmc_large_solve.txt")
 
 # the FP64 kernels of the workload's iteration (triangles, z-level windows)
-KERNEL_NAMES = {"qapply": "k_qapply_x<3, 4, double, true, 4, true>", "qprec": "k_qprec<true, 4, double, true, 24, true>"}
+KERNEL_NAMES = {"qapply": "k_qapply_x<3, 4, double, true, 4, true>",
+                "qprec": "k_qprec<true, 4, double, true, 40, true, 16, true>"}
 
 
 def log(msg: str) -> None:

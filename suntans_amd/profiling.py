@@ -31,7 +31,7 @@ COPY_BYTES = 1 << 30
 
 def short_name(name: str) -> str:
     """'void k_qapply<2, 3, 4, double, double>(sunhip::Geo, ...)' -> 'k_qapply<2, 3, 4, double, double>'."""
-    n = re.sub(r"^void ", "", name.strip())
+    n = re.sub(r"^void ", "", name.strip()).replace("(anonymous namespace)::", "")
     depth = 0
     for i, ch in enumerate(n):
         if ch == "<":
