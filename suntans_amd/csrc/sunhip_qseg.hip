@@ -8,7 +8,7 @@
 // hundred tiles leaves most of the chip idle and every wave waits out one
 // memory round trip per group of levels: 2000 columns of 50 levels took 44 us
 // for the operator and 26 us for the preconditioner, whatever the bandwidth
-// (17 and 11 us here, of which a launch alone is about 5).  Here a tile's
+// (12.7 and 8.7 us here, of which a launch alone is about 5).  Here a tile's
 // columns are loaded by up to 8 waves at once:
 //   apply    each wave forms qapply_tile's values on its segment's levels
 //   precond  each wave updates r on its levels and holds them in registers
