@@ -57,14 +57,15 @@ __global__ __launch_bounds__(256) void k_tvd_faces(Geo G, TvdArgs A, Bands B) {
 // from 6 faces (280 tiles of 67 levels 141 -> 155).
 // First-order upwind (pre false) gathers its fluxes here, and spills more the
 // more faces: triangles of up to 64 levels 500 tiles of 40 0.94 of the whole
-// columns' time, 640 1.31; quadrilaterals 239 tiles of 40 70 -> 44, 300 of 40
-// and 90 levels 71 -> 72 and 152 -> 194.
+// columns' time, 640 1.31; 319 tiles of 90 levels 129 -> 134, of 110 161 -> 146,
+// of 128 188 -> 157; quadrilaterals 239 tiles of 40 70 -> 44, 300 of 40 and 90
+// levels 71 -> 72 and 152 -> 194, 320 of 128 219 -> 227.
 template <int NF>
 static bool tvd_seg(const sunhip_grid *g, bool pre) {
   if (!g->tune_small || g->tune_tvdgrp != 2 || g->tune_tvdhead != 8) return false;
   const int ns = (g->maxdepth + SUNHIP_SEG - 1) / SUNHIP_SEG;
   if (ns < 2 || ns > (NF <= 4 ? 16 : 8) || (!pre && NF > 4)) return false;
-  if (!pre) return g->Nt <= (NF == 3 && ns <= 8 ? 512 : 256);
+  if (!pre) return g->Nt <= (NF == 3 && (ns <= 8 || ns >= 13) ? 512 : 256);
   return g->Nt <= (ns <= 8 && 8 / ns * ns >= 7 ? 768 : 512);
 }
 template <int NF, bool PRE, int SPW>

@@ -395,10 +395,10 @@ int sunhip_w_predict(sunhip_grid *g, const sunhip_wpred_params *p) {
   // The source pass sets up every face of a column per band, so its bands pay
   // up to fewer tiles the more faces: triangles, 2195 tiles of 100 levels
   // 0.70 of the whole columns' time, 3994 1.08; quadrilaterals 1497 0.7, 3993
-  // 1.13; hexagons 1497 0.86, 2198 1.04, 2998 1.15; up to 8 faces 874 0.86, 1871
-  // 1.27 (columns of 12 levels, two bands: 2994 tiles of triangles 1.1, 2198 of
+  // 1.13; hexagons 1497 0.86, 2198 1.04, 2998 1.15; up to 8 faces 874 0.86, 1246
+  // 0.96, 1526 1.22 (columns of 12 levels, two bands: 2994 tiles of triangles 1.1, 2198 of
   // hexagons 1.17)
-  const int most = g->mf <= 3 ? 2560 : g->mf == 4 ? 2048 : g->mf <= 6 ? 1536 : 1024;
+  const int most = g->mf <= 3 ? 2560 : g->mf == 4 ? 2048 : g->mf <= 6 ? 1536 : 1280;
   const bool src_bands = Bc.nb > 1 && g->Nt <= most;
   if (A.scheme) {
     int ps = prof_begin(g, PK_OTHER);
