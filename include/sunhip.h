@@ -177,7 +177,7 @@ int sunhip_q_coefficients(sunhip_grid *g);
  * the operator kernel, 8 or more; 0 whole columns), "prec_head" (top levels
  * of each column whose rows the preconditioner keeps in registers between
  * its sweeps: 0, 8, 16, 24, 32, or 40: 40 in FP64 and 48 in FP32 with
- * the next 16 in LDS; -1, the default: 40 from 1024 tiles of 64 columns up,
+ * the next 16 in LDS; -1, the default: 40 above 512 tiles of 64 columns,
  * else 0), "zreg" (1, the default: the
  * z-level windows of sunhip_set_dz; 0 off), "order" (1, the default: blocks
  * of four tiles dispatched deepest first within each XCD's run; 0 in tile

@@ -224,7 +224,7 @@ struct sunhip_grid {
                          // 2 on with a 4-waves-per-SIMD register budget, 3 on with 2 levels per group,
                          // -1 (default) by size and face count (launch_apply)
   int tune_phead = -1;   // top levels per column the preconditioner keeps in registers (0, 8, 16, 24, 32; 40:
-                         // QHead's); -1 (default) QHead's from 1024 tiles up, 0 below
+                         // QHead's); -1 (default) QHead's above SUNHIP_QSEG_FULL tiles, else 0
   int tune_band = 0;     // operator kernel over level bands of this many levels (0: whole columns)
 
   // per-kernel timing (sunhip_profile): an event pair around every launch of

@@ -441,9 +441,13 @@ int launch_prec(sunhip_grid *g, CGScal *sc, const T *coef, const T *z, T *r, T *
   // unknowns heads of 24, 32, 40 and 48 levels with 16 in LDS take 460, 421,
   // 390 and 467 us in FP64 (40: 2 waves per SIMD, 48 spills) and 231, 212,
   // 219 and 207 us in FP32; without the LDS stage 32 levels take 485 and
-  // 248 us.  Few tiles (below 1024) take the plain sweep.
+  // 248 us.  Few tiles (up to
+  // SUNHIP_QSEG_FULL) take the plain sweep; an iteration without and with the
+  // head: 720 tiles of hexagons of 100 levels 140 / 131 us, 1000 of triangles of
+  // 60 full levels 83 / 71, of random depth up to 60 and 100 levels 143 / 81 and
+  // 299 / 215.
   const bool nt = g->NT * (int64_t)sizeof(T) >= SUNHIP_STREAM_BYTES;
-  const int head = g->tune_phead < 0 ? (g->Nt >= 1024 ? QHead<T>::regs : 0)
+  const int head = g->tune_phead < 0 ? (g->Nt > SUNHIP_QSEG_FULL ? QHead<T>::regs : 0)
                                      : (g->tune_phead == 40 ? QHead<T>::regs : g->tune_phead);
   // the default head; cached stores while the vectors stay in the memory-side
   // cache (see launch_apply)

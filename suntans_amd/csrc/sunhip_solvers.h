@@ -53,12 +53,15 @@ int q_windows(sunhip_grid *g, const double *coef, const double *dzf, ZReg *Z);
 //   FP64  255 tiles of 40 levels 27 / 57 us, 508 of 70 52 / 84, 768 of 70 75 / 83,
 //         254 of hexagons of 40 32 / 74; flat: 508 of 100 110 / 115, 508 of 128
 //         143 / 158, 768 of 40 (15.8 MB) 64 / 66; but 768 of 70 (27 MB) 115 / 85,
-//         996 of 40 (20 MB) 75 / 69, 996 of 100 (51 MB) 229 / 174
+//         996 of 40 (20.4 MB) 75 / 69, 996 of 100 (51 MB) 229 / 174
+//         the line: 558 to 1000 tiles of 60 to 120 levels, any faces, 0.66 to
+//         1.03 of the whole columns' time from 15.5 to 20 MB (of 48 levels
+//         0.92 to 1.13), 0.72 to 1.33 to 24 MB, 0.9 to 1.5 beyond
 //   FP32  508 of 70 40 / 83; flat: 996 of 40 (10 MB) 54 / 62, 996 of 70 (18 MB)
 //         82 / 82, 996 of 100 (25 MB) 121 / 108
 #define SUNHIP_QSEG_FULL 512
 #define SUNHIP_QSEG_TILES 1024
-#define SUNHIP_QSEG_BYTES (16 << 20)
+#define SUNHIP_QSEG_BYTES 20000000
 bool q_seg_ok(const sunhip_grid *g, const sunhip_cg_params *prm, size_t value_bytes);
 // Whether the grid's size and dispatch order allow these kernels at all, for
 // values of value_bytes each.
