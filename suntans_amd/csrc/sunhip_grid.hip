@@ -615,10 +615,11 @@ int sunhip_grid_create(sunhip_grid **out, const sunhip_topology *T, int device) 
   if (rc) { sunhip_grid_destroy(g); return rc; }
   HIPCHK(hipMemset(g->d_count, 0, sizeof(unsigned) * 64));
   // the pinned scalars: the mirror, two polling slots and the progress word
-  // (on a cache line of its own) in one allocation
-  constexpr size_t prog_at = (3 * sizeof(CGScal) + 63) / 64 * 64;
-  HIPCHK(hipHostMalloc((void **)&g->h_sc, prog_at + 64, hipHostMallocDefault));
-  g->h_poll = g->h_sc + 1;
+  // in one allocation, on cache lines of their own
+  constexpr size_t poll_at = (sizeof(CGScal) + 127) / 128 * 128;
+  constexpr size_t prog_at = poll_at + (2 * sizeof(CGScal) + 127) / 128 * 128;
+  HIPCHK(hipHostMalloc((void **)&g->h_sc, prog_at + 128, hipHostMallocDefault));
+  g->h_poll = (CGScal *)((char *)g->h_sc + poll_at);
   g->h_prog = (unsigned long long *)((char *)g->h_sc + prog_at);
   *g->h_prog = 0;
   HIPCHK(hipEventCreateWithFlags(&g->evp[0], hipEventDisableTiming));
