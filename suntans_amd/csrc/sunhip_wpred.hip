@@ -393,12 +393,14 @@ int sunhip_w_predict(sunhip_grid *g, const sunhip_wpred_params *p) {
   const Bands Bc = level_bands(g, g->Nt), Be = level_bands(g, g->Net);
   const int ncb = (g->Nt * Bc.nb + 3) / 4;
   // The source pass sets up every face of a column per band, so its bands pay
-  // up to fewer tiles the more faces: triangles, 2195 tiles of 100 levels
-  // 0.70 of the whole columns' time, 3994 1.08; quadrilaterals 1497 0.7, 3993
-  // 1.13; hexagons 1497 0.86, 2198 1.04, 2998 1.15; up to 8 faces 874 0.86, 1246
-  // 0.96, 1526 1.22 (columns of 12 levels, two bands: 2994 tiles of triangles 1.1, 2198 of
-  // hexagons 1.17)
-  const int most = g->mf <= 3 ? 2560 : g->mf == 4 ? 2048 : g->mf <= 6 ? 1536 : 1280;
+  // up to fewer tiles the more faces.  Bands against whole columns, smooth
+  // depths: triangles of 100 levels, 2692 tiles 325 us / 444, 3200 367 / 476, 3906
+  // 506 / 494; quadrilaterals of 60 levels, 2698 290 / 335, 3300 380 / 366;
+  // hexagons of 60, 1697 349 / 412, 2198 455 / 448.  With depths at random they
+  // meet earlier: triangles at 2994 tiles (1.00 of the time, 12 levels 1.1),
+  // quadrilaterals at 2198 (0.96 to 1.07), hexagons at 1497 to 2198 (0.86, 1.04),
+  // up to 8 faces at 1246 (0.96; 1526 1.22)
+  const int most = g->mf <= 3 ? 3328 : g->mf == 4 ? 2816 : g->mf <= 6 ? 2048 : 1280;
   const bool src_bands = Bc.nb > 1 && g->Nt <= most;
   if (A.scheme) {
     int ps = prof_begin(g, PK_OTHER);
